@@ -465,8 +465,7 @@ __device__ __forceinline__ float minps1(float a, float b) { return a < b ? a : b
 __device__ __forceinline__ float exp_cephes(float x) {
     constexpr float P[6] = { 1.9875691500e-4f, 1.3981999507e-3f, 8.3334519073e-3f,
                              4.1665795894e-2f, 1.6666665459e-1f, 5.0000001201e-1f };
-    x = minps1(x, 88.3762626647949f);
-    x = maxps1(x, -87.3f);
+    x = __builtin_fmaxf(__builtin_fminf(x, 88.3762626647949f), -87.3f);
     const float n = __builtin_rintf(x * 1.44269504088896341f);
     float r = __builtin_fmaf(-n, 0.693359375f, x);
     r = __builtin_fmaf(-n, -2.12194440e-4f, r);
@@ -475,8 +474,7 @@ __device__ __forceinline__ float exp_cephes(float x) {
 #pragma unroll
     for (int i = 1; i < 6; ++i) p = __builtin_fmaf(p, r, P[i]);
     p = __builtin_fmaf(p, r2, r + 1.0f);
-    const uint32_t e = (uint32_t) ((int) n + 127) << 23;
-    return p * __uint_as_float(e);
+    return __builtin_ldexpf(p, (int) n);
 }
 
 // op_gate (src/nexterabert.cpp:507-522, AVX2 path; C % 8 == 0): sigmoid(g) * y with
@@ -675,6 +673,25 @@ __global__ __launch_bounds__(256) void produce_quantize_kernel(Src src, int T, i
     quantize_block<ACT_MAX>(src, T, n_in, KS, n_blk, q, sx, g, B, stage);
 }
 
+// This lane's number, computed where it is used: an asm the compiler cannot hoist, so
+// that values derived from it are not kept live across a loop (register pressure).
+__device__ __forceinline__ int lane_here() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+
+// A raw buffer resource over `bytes` bytes at `base` (gfx9 descriptor word 3): buffer
+// loads take a scalar base, a scalar offset and one vector offset, so that a wave's
+// address arithmetic stays on the scalar unit, and they count in vmcnt only.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void * base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short) 0, (int) bytes, 0x00020000);
+}
+// 16 bytes per lane at byte soff (wave-uniform) + voff (per lane) of the buffer.
+__device__ __forceinline__ v4i bload16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, (int) voff, (int) soff, 0);
+}
+
 // ---------------------------------------------------------------------------
 // Attention (head_dim 64) inside each document of a packed layout
 // ---------------------------------------------------------------------------
@@ -823,56 +840,517 @@ __global__ __launch_bounds__(64) void attention_kernel(attn_params p) {
     o[lane] = acc;
 }
 
-// softmax_exp (src/nexterabert.cpp:177-200) for one (query, head) pair whose n scores sit in
-// LDS at Sp, by the 16 lanes sk of the pair (one wave's 16-lane group), in three steps with a
-// workgroup barrier between them (the callers hold it):
-//   softmax_max_exp   m (a NaN first score wins, else the largest score), then exp256(s - m)
-//                     in place for the n & ~7 grouped keys and the C library's expf for the rest
-//   softmax_inv       lanes l < 8 add keys 8i + l in order of i, hsum256 over the 8 lanes, the
-//                     tail keys added after in order; returns 1 / sum (on lane 0 of the group)
-//   softmax_weights   w = e * (1 / sum) in place
-// Loads are issued 16 at a time ahead of the adds that consume them in order.
-__device__ __forceinline__ void softmax_max_exp(float * Sp, int n, int sk) {
-    const int ng = n & ~7;
-    const float s0 = Sp[0];
-    float mx = -__builtin_inff();
-#pragma unroll 8
-    for (int j = sk; j < n; j += 16) mx = fmaxf(mx, Sp[j]);
-#pragma unroll
-    for (int sft = 8; sft >= 1; sft >>= 1) mx = fmaxf(mx, __shfl_xor(mx, sft));
-    const float m = __builtin_isnan(s0) ? s0 : mx;
-#pragma unroll 8
-    for (int j = sk; j < ng; j += 16) Sp[j] = exp_cephes(Sp[j] - m);
-    for (int j = ng + sk; j < n; j += 16) Sp[j] = expf_libm(Sp[j] - m);
+__device__ __forceinline__ bool finite4(const v4f & x) {
+    return __builtin_isfinite(x.x) && __builtin_isfinite(x.y) && __builtin_isfinite(x.z) && __builtin_isfinite(x.w);
 }
 
-__device__ __forceinline__ float softmax_inv(const float * Sp, int n, int sk, bool active) {
-    const int ng = n & ~7;
-    float ls = 0.0f;
-    if (active && sk < 8) {
-        int j = sk;
-        for (; j + 8 * 15 < ng; j += 8 * 16) {
-            float v[16];
-#pragma unroll
-            for (int u = 0; u < 16; ++u) v[u] = Sp[j + 8 * u];
-#pragma unroll
-            for (int u = 0; u < 16; ++u) ls = ls + v[u];
+// ---------------------------------------------------------------------------
+// Attention on the matrix cores, bit for bit attention_kernel's operations.
+//
+// v_mfma_f32_16x16x4_f32 computes each output as four fused multiply-adds in order of k, each
+// rounded once (0 mismatches against fmaf chains in 1.6 M outputs over the whole exponent
+// range, subnormals and signed zeros among them). So both of the reference's fp32 chains
+// run on it exactly:
+//   scores   chain l of a dot product is q[l] k[l], then fma(q[8c + l], k[8c + l], a_l) for
+//            c = 1..7: with lane group c (lane >> 4) of the operands holding elements 8c + l, one
+//            MFMA does c = 0..3 of chain l from -0 (fma(q, k, -0) rounds and signs as q * k),
+//            a second c = 4..7; the 8 chains of a score end in one lane for the tree
+//   values   acc = fma(w_j, v_j[d], acc) over the keys in order: one MFMA takes four keys
+// A workgroup takes the ATT_P (query, head) pairs of ATT_P / rep consecutive query rows and one
+// KV head; a tile is 16 keys. Scores are computed transposed (keys are the MFMA's rows) with row
+// 4g + r standing for key 4r + g, so that register r of lane (g = lane >> 4, pair = lane & 15)
+// is the score of key 4r + g: what every later phase wants without moving data between lanes:
+//   scores   the waves take the tiles in turn, 16 MFMAs each; a tile's 4 scores per lane are
+//            stored as 16 bytes per lane (1 KiB per tile, in LDS; past lds_tiles in the
+//            workgroup's slot of the workspace)
+//   softmax  each wave takes its own tiles again: exponentials in place. Keys of one lane are
+//            4 apart, so the accumulators of softmax_exp (element i of lane sum l is key 8i + l)
+//            are two per lane, registers 0, 2 and 1, 3, whatever key the pair's first is; one
+//            wave adds them over all tiles in order, hsum256 is their sum, then lanes 32 and 16
+//            apart; the tail keys' e (kept apart) follow in order
+//   values   register r, times 1 / sum, is the MFMA's A operand of keys 4r .. 4r + 3; the waves
+//            take 16 of the 64 dimensions each, all tiles
+// A tile is clean when every active pair attends to all its keys, none of them a pair's first or
+// in its last n % 8; others compute both trees and mask. Keys outside a pair's range get e = -0
+// (its products with finite values leave acc as it is); where an output is Inf or NaN the keys are
+// taken again one by one, each result kept only for the pairs that attend to the key.
+// Key and value rows come straight from memory (each is read once per workgroup) by buffer
+// loads that return 0 past the last key, whole lines to a few lanes, and turn into operand order
+// through a little LDS of the wave's own: a load whose neighbouring lanes are on different lines
+// takes a cycle a lane.
+// Pairs are processed together while the keys they attend to span at most the tiles there are,
+// else document by document.
+// ---------------------------------------------------------------------------
+constexpr int ATT_P = 16;              // (query, head) pairs per workgroup
+constexpr int ATT_TILE = 16;           // keys per tile
+constexpr int ATT_TILE_BYTES = ATT_P * ATT_TILE * 4;
+constexpr int ATT_VC = 4;              // tiles per step of the value loop
+constexpr int ATT_STATIC_LDS = 9216;   // LDS beside the tiles, at most
+constexpr int ATT_MAX_KEYS = 1 << 23;  // keys whose row offsets fit the buffer loads' 32 bits
+
+// the workspace is 4-byte aligned
+typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));
+
+// min / max over the 16 lanes of a row of lanes (the rows agree), by DPP row rotations
+template <typename F>
+__device__ __forceinline__ int row_fold(int x, F f) {
+    x = f(x, __builtin_amdgcn_update_dpp(x, x, 0x128, 0xf, 0xf, false));
+    x = f(x, __builtin_amdgcn_update_dpp(x, x, 0x124, 0xf, 0xf, false));
+    x = f(x, __builtin_amdgcn_update_dpp(x, x, 0x122, 0xf, 0xf, false));
+    x = f(x, __builtin_amdgcn_update_dpp(x, x, 0x121, 0xf, 0xf, false));
+    return __builtin_amdgcn_readfirstlane(x);
+}
+__device__ __forceinline__ int row_min(int x) {
+    return row_fold(x, [](int a, int b) { return min(a, b); });
+}
+__device__ __forceinline__ int row_max(int x) {
+    return row_fold(x, [](int a, int b) { return max(a, b); });
+}
+
+// doc_of for the lanes of a wave, whose rows t start at the wave's t0 and rise by a few: t0's
+// document by 64 offsets at a time, then each lane's own.
+__device__ __forceinline__ doc_rows doc_of_wave(const int32_t * cu, int n, int t0, int t, int T, int lane) {
+    int a = 0, len = n;
+    while (len > 64) {
+        const int step = (len + 63) >> 6, m = lane * step;
+        const int c = __popcll(__ballot(m < len && cu[a + min(m, len - 1)] <= t0));
+        const int skip = max(c - 1, 0) * step;
+        a += skip;
+        len = min(step, len - skip);
+    }
+    a += max(__popcll(__ballot(lane < len && cu[a + min(lane, len - 1)] <= t0)) - 1, 0);
+    while (a + 1 < n && cu[a + 1] <= t) ++a;
+    doc_rows r;
+    r.d = a;
+    r.lo = min(max(cu[a], 0), T);
+    r.hi = min(max(cu[a + 1], r.lo), T);
+    return r;
+}
+
+// Keeps the compiler from moving memory operations across: loads stay where they are issued ahead
+// of their use, and a wave's LDS writes before its later reads by other lanes (LDS serves a
+// wave's operations in order).
+__device__ __forceinline__ void keep_order() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ v4f bload16f(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
+    return __builtin_bit_cast(v4f, bload16(r, voff, 0));
+}
+
+// WS: tiles past lds_tiles (a multiple of ATT_VC) live in the workgroup's slot of ws (ws_tiles
+// tiles each), and the grid is persistent.
+//
+// What bounds it: an fp32 MFMA (32 cycles for 1,024 FMAs) keeps the vector unit's FMA rate, and
+// vector instructions do not hide under it (16 MFMAs with 2 or 8 vector instructions each on four
+// waves: 38.6 and 57 cycles per MFMA against 32.6), so a tile costs a SIMD at least 32 x 32 cycles
+// and ~140 vector instructions of ~2.5, about 1,400. The matrix cores take the operands' traffic
+// and issue slots away: the same FMAs as vector
+// instructions, with their LDS reads and broadcasts, ran at about 30 TFLOP/s; this runs at 45-65. At most 128
+// registers, so that four workgroups share a CU: two took 181 us where four take 161 (8 x 1,024
+// tokens, band 256). Before -> now: 1,024 keys 178 -> 101 us, 8 x 1,024 tokens in bands of
+// 257 keys 279 -> 174 us, 32 documents of 16 to 2,048 tokens 7.45 -> 3.02 ms (with the launch).
+// Lane numbers are taken anew in each phase: kept across them, the addresses made from them cost
+// 50 registers.
+template <bool WS>
+__global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, int lds_tiles, int ws_tiles,
+                                                                           float * __restrict__ ws) {
+    extern __shared__ __attribute__((aligned(16))) float att_lds[];
+    __shared__ __attribute__((aligned(16))) float wbuf[4][512];   // each wave's own: keys or values in transit
+    __shared__ float mx_s[4][ATT_P], s0_s[ATT_P], inv_s[ATT_P], tail_s[ATT_P][8];
+    const int lane = (int) threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+    const int g4 = lane >> 4, pi = lane & 15;
+    const int lg_rep = __builtin_ctz((unsigned) (p.H / p.G)), rep = 1 << lg_rep, nq = ATT_P >> lg_rep;
+    const int n_tiles = p.G * ((p.T + nq - 1) / nq);
+    const int cap = ATT_TILE * (lds_tiles + ws_tiles);
+    // the wave that adds up: waves 0 of a CU's workgroups share a SIMD, so it goes by their slot
+    // there (hwreg HW_ID's wave slot, 4 bits at 0)
+    __shared__ int adder_s;
+    if (threadIdx.x == 0) adder_s = __builtin_amdgcn_s_getreg(4 | (0 << 6) | (3 << 11)) & 3;
+    float * const slot = WS ? ws + (size_t) blockIdx.x * ws_tiles * (ATT_TILE_BYTES / 4) : nullptr;
+    // float x of tile i's scores, in LDS or in the slot
+    auto in_lds = [&](int i, int x) -> float * { return att_lds + i * 256 + x; };
+    auto in_slot = [&](int i, int x) -> float * { return slot + (size_t) (i - lds_tiles) * 256 + x; };
+    // a lane's 4 scores of a tile known to be in LDS (lds_tag) or in the slot (slot_tag), or of any
+    struct lds_tag {};
+    struct slot_tag {};
+    auto t_load = [&](auto tag, int i, int x) -> v4f {
+        if constexpr (std::is_same_v<decltype(tag), lds_tag>) return *reinterpret_cast<const v4f *>(in_lds(i, x));
+        else return *reinterpret_cast<const v4f_u *>(in_slot(i, x));
+    };
+    auto t_store = [&](auto tag, int i, int x, v4f e) {
+        if constexpr (std::is_same_v<decltype(tag), lds_tag>) *reinterpret_cast<v4f *>(in_lds(i, x)) = e;
+        else *reinterpret_cast<v4f_u *>(in_slot(i, x)) = e;
+    };
+    auto s_load = [&](int i, int x) -> v4f {
+        return !WS || i < lds_tiles ? t_load(lds_tag{}, i, x) : t_load(slot_tag{}, i, x);
+    };
+    auto s_store = [&](int i, int x, v4f e) {
+        if (!WS || i < lds_tiles) t_store(lds_tag{}, i, x, e);
+        else t_store(slot_tag{}, i, x, e);
+    };
+
+    for (int bt = (int) blockIdx.x; bt < n_tiles; bt += (int) gridDim.x) {
+        // the KV head changes fastest: with 8 of them each XCD's L2 serves one
+        const int g = bt % p.G, t0 = (bt / p.G) * nq;
+        const int t = t0 + (pi >> lg_rep), h = (g << lg_rep) + (pi & (rep - 1));
+        doc_rows dr = doc_of_wave(p.cu, p.n_seqs, t0, min(t, p.T - 1), p.T, lane);
+        if (p.half >= 0) {
+            dr.lo = max(dr.lo, t - p.half);
+            dr.hi = (int) min((long long) dr.hi, (long long) t + p.half + 1);
         }
-        for (; j < ng; j += 8) ls = ls + Sp[j];
-    }
-    ls = ls + __shfl_xor(ls, 4);                           // lanes 8..15 hold 0 and stay among themselves
-    ls = ls + __shfl_xor(ls, 2);
-    ls = ls + __shfl_xor(ls, 1);
-    float sum = ls;
-    if (active && sk == 0) {
-        for (int j = ng; j < n; ++j) sum = sum + Sp[j];
-    }
-    return 1.0f / sum;
-}
+        const int lo = dr.lo, hi = dr.hi, n = hi - lo;
+        const bool valid = t < p.T && n > 0 && n <= p.max_keys;
+        const float scale = p.scale[dr.d];
+        if (t < p.T && !valid) {                           // no keys, or more than max_keys
+            const float nan = __uint_as_float(0x7fc00000u);
+            *reinterpret_cast<v4f_u *>(p.out + (size_t) t * p.H * 64 + (size_t) h * 64 + 16 * w + 4 * g4) =
+                v4f{ nan, nan, nan, nan };
+        }
 
-__device__ __forceinline__ void softmax_weights(float * Sp, int n, int sk, float inv) {
-#pragma unroll 8
-    for (int j = sk; j < n; j += 16) Sp[j] = Sp[j] * inv;
+        bool todo = valid;
+        while (__any(todo)) {                              // the same in every wave
+            bool act = todo;
+            int kl = row_min(act ? lo : INT_MAX), kh = row_max(act ? hi : INT_MIN);
+            if (kh - kl > cap) {
+                const int d0 = row_min(todo ? dr.d : INT_MAX);
+                act = todo && dr.d == d0;
+                kl = row_min(act ? lo : INT_MAX);
+                kh = row_max(act ? hi : INT_MIN);
+            }
+            const int na = act ? n : 0, ng = na & ~7;
+            const int nt = (kh - kl + ATT_TILE - 1) / ATT_TILE;
+            // clean tiles [c0, c1): past every pair's first key's tile, before any pair's tail keys or end
+            int c0 = (row_max(act ? lo : INT_MIN) - kl) / ATT_TILE + 1;
+            int c1 = (row_min(act ? lo + ng : INT_MAX) - kl) / ATT_TILE;
+            if (c1 <= c0) c0 = c1 = 0;
+            const int n_edge = nt - (c1 - c0);             // the others, [0, c0) and [c1, nt), taken by number
+            auto edge = [&](int d) { return d < c0 ? d : d - c0 + c1; };
+            const uint32_t kv_bytes = (uint32_t) (kh - kl) * 256u;
+
+            // scores
+            {
+                const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane;
+                const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(p.k + ((size_t) g * p.T + kl) * 64, kv_bytes);
+                // row (of the MFMA) 8 (k & 1) + (lane >> 3), its 16-byte piece (lane & 7) + 8 (k >> 1)
+                const int fr = lane >> 3, fc = lane & 7;
+                const uint32_t koff0 = (uint32_t) (4 * (fr & 3) + (fr >> 2)) * 256u + (uint32_t) fc * 16u;
+                // a half row's pieces at slot (row ^ row >> 3), piece ^ (row & 7): neither the writes
+                // (8 lanes a row) nor the reads (a row per lane) meet on a bank
+                float * const kw0 = wbuf[w] + fr * 32 + (fc ^ fr) * 4;
+                float * const kw1 = wbuf[w] + ((8 + fr) ^ 1) * 32 + (fc ^ fr) * 4;
+                const float * const kr0 = wbuf[w] + (pi ^ (pi >> 3)) * 32 + ((2 * g4) ^ (pi & 7)) * 4;
+                const float * const kr1 = wbuf[w] + (pi ^ (pi >> 3)) * 32 + ((2 * g4 + 1) ^ (pi & 7)) * 4;
+                const float * const qrow = p.q + (size_t) min(t0 + (pi >> lg_rep), p.T - 1) * p.H * 64 +
+                                           (size_t) ((g << lg_rep) + (pi & (rep - 1))) * 64 + 8 * g4;
+                v4f qf[4];
+                qf[0] = *reinterpret_cast<const v4f_u *>(qrow);
+                qf[1] = *reinterpret_cast<const v4f_u *>(qrow + 4);
+                qf[2] = *reinterpret_cast<const v4f_u *>(qrow + 32);
+                qf[3] = *reinterpret_cast<const v4f_u *>(qrow + 36);
+                const int key0 = kl + g4 - lo;             // key 4r + g4 of tile i is the pair's key0 + 16 i + 4 r
+                float mx = -__builtin_inff();
+                v4f raw[4];
+                auto fetch = [&](int i) {
+                    uint32_t o = koff0 + (uint32_t) i * 4096u;
+                    asm volatile("" : "+v"(o));            // one offset register, the rest immediate
+                    raw[0] = bload16f(kr, o);
+                    raw[1] = bload16f(kr, o + 512);
+                    raw[2] = bload16f(kr, o + 128);
+                    raw[3] = bload16f(kr, o + 640);
+                    keep_order();
+                };
+                auto turn = [&](v4f (&kf)[4]) {            // raw -> operand order, half rows in turn
+                    *reinterpret_cast<v4f *>(kw0) = raw[0];
+                    *reinterpret_cast<v4f *>(kw1) = raw[1];
+                    keep_order();
+                    kf[0] = *reinterpret_cast<const v4f *>(kr0);
+                    kf[1] = *reinterpret_cast<const v4f *>(kr1);
+                    keep_order();
+                    *reinterpret_cast<v4f *>(kw0) = raw[2];
+                    *reinterpret_cast<v4f *>(kw1) = raw[3];
+                    keep_order();
+                    kf[2] = *reinterpret_cast<const v4f *>(kr0);
+                    kf[3] = *reinterpret_cast<const v4f *>(kr1);
+                    keep_order();
+                };
+                auto chains = [&](const v4f (&kf)[4], v4f (&a)[8]) {
+                    const v4f nz = { -0.0f, -0.0f, -0.0f, -0.0f };
+#pragma unroll
+                    for (int l = 0; l < 8; ++l)
+                        a[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[l >> 2][l & 3], qf[l >> 2][l & 3], nz, 0, 0, 0);
+#pragma unroll
+                    for (int l = 0; l < 8; ++l)
+                        a[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[2 + (l >> 2)][l & 3], qf[2 + (l >> 2)][l & 3], a[l], 0, 0, 0);
+                };
+                auto tree = [&](const v4f (&a)[8]) {
+                    v4f s;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        s[r] = (((a[0][r] + a[1][r]) + (a[2][r] + a[3][r])) + ((a[4][r] + a[5][r]) + (a[6][r] + a[7][r]))) * scale;
+                    return s;
+                };
+                auto tile = [&](const v4f (&kf)[4], int i) {
+                    v4f a[8];
+                    chains(kf, a);
+                    const v4f s = tree(a);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[r]);
+                    s_store(i, lx, s);
+                };
+                v4f ka[4];
+                if (c0 + w < c1) {
+                    fetch(c0 + w);
+#pragma unroll 1
+                    for (int i = c0 + w; i < c1; i += 4) {
+                        turn(ka);
+                        fetch(i + 4);
+                        tile(ka, i);
+                    }
+                }
+#pragma unroll 1
+                for (int d = 3 - w; d < n_edge; d += 4) {
+                    const int i = edge(d);
+                    fetch(i);
+                    turn(ka);
+                    v4f a[8];
+                    chains(ka, a);
+                    v4f s = tree(a);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int jr = key0 + ATT_TILE * i + 4 * r;
+                        const float st = (((a[0][r] + a[4][r]) + (a[2][r] + a[6][r])) + ((a[1][r] + a[5][r]) + (a[3][r] + a[7][r]))) * scale;
+                        if (jr >= ng) s[r] = st;
+                        if (jr >= 0 && jr < na) mx = fmaxf(mx, s[r]);
+                        if (act && jr == 0) s0_s[pi] = s[r];
+                    }
+                    s_store(i, lx, s);
+                }
+                mx = fmaxf(mx, __shfl_xor(mx, 16));
+                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                if (lane < ATT_P) mx_s[w][pi] = mx;
+            }
+            __syncthreads();
+
+            // exponentials: m is NaN if the first score is, else the largest score that is not NaN.
+            // Tail keys keep their scores in the tiles here; the C library's expf takes them, one
+            // key j of a pair per lane of waves 2 and 3.
+            {
+                const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane;
+                const float s0 = s0_s[pi];
+                const float mx = fmaxf(fmaxf(mx_s[0][pi], mx_s[1][pi]), fmaxf(mx_s[2][pi], mx_s[3][pi]));
+                const float m = __builtin_isnan(s0) ? s0 : mx;
+                const int key0 = kl + g4 - lo;
+                auto part = [&](auto tag, int a, int b) {  // tiles a, a + 4, ... below b
+                    if (a >= b) return;
+                    const int last = a + ((b - 1 - a) & ~3);
+                    v4f x[2], y[2];
+                    x[0] = t_load(tag, a, lx);
+                    x[1] = t_load(tag, min(a + 4, last), lx);
+                    for (int i = a; i < b; i += 8) {
+                        y[0] = t_load(tag, min(i + 8, last), lx);
+                        y[1] = t_load(tag, min(i + 12, last), lx);
+                        keep_order();
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) x[u][r] = exp_cephes(x[u][r] - m);
+                        t_store(tag, i, lx, x[0]);
+                        if (i + 4 < b) t_store(tag, i + 4, lx, x[1]);
+                        x[0] = y[0];
+                        x[1] = y[1];
+                    }
+                };
+                if constexpr (WS) {
+                    const int cl = min(max(c0, lds_tiles), c1);
+                    part(lds_tag{}, c0 + w, cl);
+                    part(slot_tag{}, cl + ((c0 + w - cl) & 3), c1);
+                } else {
+                    part(lds_tag{}, c0 + w, c1);
+                }
+                const int j = 4 * (w & 1) + g4;
+                if (w >= 2 && j < na - ng) {
+                    const int k = lo - kl + ng + j, x = ((k & 3) * 16 + pi) * 4 + ((k & 15) >> 2);
+                    const float s = !WS || k / ATT_TILE < lds_tiles ? *in_lds(k / ATT_TILE, x) : *in_slot(k / ATT_TILE, x);
+                    tail_s[pi][j] = expf_libm(s - m);
+                }
+#pragma unroll 1
+                for (int d = 3 - w; d < n_edge; d += 4) {
+                    const int i = edge(d);
+                    v4f e = s_load(i, lx);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int jr = key0 + ATT_TILE * i + 4 * r;
+                        const float x = exp_cephes(e[r] - m);
+                        if (jr < ng) e[r] = jr >= 0 ? x : -0.0f;
+                        else if (jr >= na) e[r] = -0.0f;
+                    }
+                    s_store(i, lx, e);
+                }
+            }
+            // the first values, under way meanwhile
+            const __amdgpu_buffer_rsrc_t vr = buffer_rsrc(p.v + ((size_t) g * p.T + kl) * 64, kv_bytes);
+            // a tile's 16 dimensions of this wave: key lane >> 2, 16-byte piece lane & 3
+            const int vlane = lane_here();
+            const uint32_t voff = (uint32_t) (vlane >> 2) * 256u + (uint32_t) w * 64u + (uint32_t) (vlane & 3) * 16u;
+            v4f va[ATT_VC], vb[ATT_VC], ea[ATT_VC], eb[ATT_VC];
+            auto v_fetch = [&](v4f (&v)[ATT_VC], int i0) {
+#pragma unroll
+                for (int u = 0; u < ATT_VC; ++u) {
+                    uint32_t o = voff + (uint32_t) (i0 + u) * 4096u;
+                    asm volatile("" : "+v"(o));
+                    v[u] = bload16f(vr, o);
+                }
+                keep_order();
+            };
+            auto e_fetch = [&](auto tag, v4f (&e)[ATT_VC], int i0, int last, int lx) {
+#pragma unroll
+                for (int u = 0; u < ATT_VC; ++u) e[u] = t_load(tag, min(i0 + u, last), lx);
+                keep_order();
+            };
+            v_fetch(va, 0);
+            __syncthreads();
+
+            // 1 / sum
+            if (w == adder_s) {
+                const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane;
+                const int key0 = kl + g4 - lo;             // key 4r + g4 of tile i is the pair's key0 + 16 i + 4 r
+                float l0 = 0.0f, l1 = 0.0f;
+                auto add = [&](const v4f & e) { l0 = l0 + e.x; l1 = l1 + e.y; l0 = l0 + e.z; l1 = l1 + e.w; };
+                auto add_edges = [&](int a, int b) {       // without the tail keys
+#pragma unroll 1
+                    for (int i = a; i < b; ++i) {
+                        v4f e = s_load(i, lx);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (key0 + ATT_TILE * i + 4 * r >= ng) e[r] = 0.0f;
+                        add(e);
+                    }
+                };
+                auto part = [&](auto tag, int a, int b) {
+                    int i = a;
+                    if (i + 2 * ATT_VC <= b) {
+                        e_fetch(tag, ea, i, b - 1, lx);
+                        for (; i + 2 * ATT_VC <= b; i += 2 * ATT_VC) {
+                            e_fetch(tag, eb, i + ATT_VC, b - 1, lx);
+#pragma unroll
+                            for (int u = 0; u < ATT_VC; ++u) add(ea[u]);
+                            e_fetch(tag, ea, i + 2 * ATT_VC, b - 1, lx);
+#pragma unroll
+                            for (int u = 0; u < ATT_VC; ++u) add(eb[u]);
+                        }
+                    }
+                    for (; i < b; ++i) add(t_load(tag, i, lx));
+                };
+                add_edges(0, c0);
+                if constexpr (WS) {
+                    const int cl = min(max(c0, lds_tiles), c1);
+                    part(lds_tag{}, c0, cl);
+                    part(slot_tag{}, cl, c1);
+                } else {
+                    part(lds_tag{}, c0, c1);
+                }
+                add_edges(c1, nt);
+                float sum = l0 + l1;
+                sum = sum + __shfl_xor(sum, 32);
+                sum = sum + __shfl_xor(sum, 16);
+                for (int j = 0; j < na - ng; ++j) {
+                    const float e = tail_s[pi][j];
+                    sum = sum + e;
+                    const int k = lo - kl + ng + j, x = ((k & 3) * 16 + pi) * 4 + ((k & 15) >> 2);
+                    if (g4 == 0) *(!WS || k / ATT_TILE < lds_tiles ? in_lds(k / ATT_TILE, x) : in_slot(k / ATT_TILE, x)) = e;
+                }
+                if (lane < ATT_P) inv_s[pi] = 1.0f / sum;
+            }
+            __syncthreads();
+
+            // values
+            {
+                const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane;
+                const float inv = inv_s[pi];
+                v4f acc = { 0.0f, 0.0f, 0.0f, 0.0f };
+                // two tiles at a time through the wave's buffer: register r of a tile is key 4r + g4,
+                // dimension 16 w + pi
+                auto turn = [&](v4f (&v)[ATT_VC]) {
+#pragma unroll
+                    for (int u = 0; u < ATT_VC; u += 2) {
+                        *reinterpret_cast<v4f *>(wbuf[w] + lane * 4) = v[u];
+                        *reinterpret_cast<v4f *>(wbuf[w] + 256 + lane * 4) = v[u + 1];
+                        keep_order();
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            v[u][r] = wbuf[w][64 * r + lane];
+                            v[u + 1][r] = wbuf[w][256 + 64 * r + lane];
+                        }
+                        keep_order();
+                    }
+                };
+                // tiles past the last: weight -0, value 0
+                auto tiles = [&](const v4f (&e)[ATT_VC], const v4f (&v)[ATT_VC], int i) {
+#pragma unroll
+                    for (int u = 0; u < ATT_VC; ++u) {
+                        const v4f wt = e[u] * (i + u < nt ? inv : -0.0f);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[r], v[u][r], acc, 0, 0, 0);
+                    }
+                };
+                turn(va);
+                v_fetch(vb, ATT_VC);
+                int i = 0;
+                auto part = [&](auto tag, int b) {
+                    if (i >= b) return;
+                    e_fetch(tag, ea, i, b - 1, lx);
+                    for (; i < b; i += ATT_VC) {
+                        e_fetch(tag, eb, i + ATT_VC, b - 1, lx);
+                        tiles(ea, va, i);
+#pragma unroll
+                        for (int u = 0; u < ATT_VC; ++u) { va[u] = vb[u]; ea[u] = eb[u]; }
+                        turn(va);
+                        v_fetch(vb, i + 2 * ATT_VC);
+                    }
+                };
+                if constexpr (WS) {
+                    part(lds_tag{}, min(lds_tiles, nt));
+                    part(slot_tag{}, nt);
+                } else {
+                    part(lds_tag{}, nt);
+                }
+                const uint32_t rows = (uint32_t) __ballot(act) & 0xffffu;
+                auto is_act = [&](int r) { return ((rows >> (4 * g4 + r)) & 1) != 0; };
+                bool bad = false;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bad = bad || (is_act(r) && !__builtin_isfinite(acc[r]));
+                // an Inf or NaN value makes every pair's sum of its dimension Inf or NaN, whatever the
+                // weights, also for pairs that do not attend to it: key by key then
+                if (__any(bad)) {
+                    acc = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll 1
+                    for (int j = 0; j < ATT_TILE * nt; ++j) {
+                        const v4f e = s_load(j / ATT_TILE, lx) * inv;
+                        const int r = (j & 15) >> 2;
+                        const bool mine = (j & 3) == g4;
+                        const float wj = r < 2 ? (r == 0 ? e.x : e.y) : (r == 2 ? e.z : e.w);
+                        const float vj = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                            vr, (int) ((uint32_t) j * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0));
+                        const v4f one = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? wj : 0.0f, mine ? vj : -0.0f, acc, 0, 0, 0);
+                        const uint64_t in = __ballot(act && kl + j >= lo && kl + j < hi);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            if ((in >> (4 * g4 + k)) & 1) acc[k] = one[k];
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int pr = 4 * g4 + r;
+                    if (is_act(r))
+                        p.out[(size_t) (t0 + (pr >> lg_rep)) * p.H * 64 + (size_t) ((g << lg_rep) + (pr & (rep - 1))) * 64 + 16 * w + pi] = acc[r];
+                }
+            }
+            todo = todo && !act;
+            __syncthreads();                               // the scores and sums have been read
+        }
+    }
 }
 
 // acc[i] = fma(w_i[lane L of this lane's 16-lane row], v_L, acc[i]) for i < 4 and the 16 keys
@@ -900,29 +1378,6 @@ __device__ __forceinline__ void fmac_bcast4_16(float (&acc)[4], const float (&w)
 }
 #undef NXG_FB4
 
-// The same attention for a tile of (query, head) pairs: the ATT_P pairs of one workgroup are
-// ATT_P / rep consecutive query rows times the rep query heads of one KV head, so that every
-// key and value row read into LDS serves all of them. Per pair the operations and their
-// order are attention_kernel's (the reference's scores_d64, softmax_exp, values_d64):
-//   scores    the 8 FMA chains (a_l = q[l] k[l], then fma(q[8c+l], k[8c+l], a_l) for
-//             c = 1..7) and the HADD tree (keys of whole groups of 8) or hsum256's (the last
-//             n % 8 keys) in registers, times the scale; kept in LDS, [pair][key - the pair's
-//             first key]. Chain-parallel: 8 lanes per key, each one chain of 16 pairs
-//             (WIDE, 128 query registers, chosen when the scores' LDS already limits a CU to
-//             two workgroups) or of 8 pairs (64 registers), so that a staged key row is read
-//             from LDS once for 16 or 8 pairs (att_chain_tree)
-//   softmax   16 threads per pair: the maximum (a NaN first score wins), exp256 / the C
-//             library's expf in place, then threads l < 8 add the keys 8i + l in order of i
-//             (the 8 lanes of softmax_exp's accumulator) and hsum256 over them, the tail keys
-//             added after; each weight becomes w * (1 / sum)
-//   values    thread (dim d, 4 pairs): acc = fma(w_j, v_j[d], acc) over the keys in order;
-//             a tile's weights of a pair are read once, key j0 + 16h + k in lane k of every
-//             16-lane row of register h, and each fma takes its weight through DPP row_newbcast
-//             (keys outside a pair's range with weight 0, adding fma(0, v, acc) = acc; readlane
-//             and a per-key range test on tiles whose staged values hold an Inf or NaN), so the
-//             key loop reads only v_j[d] from LDS.
-// Keys are staged ATT_KT at a time ([key][ATT_KS] floats; the padding puts the 16 rows one
-// wave reads on different banks). Pairs whose keys exceed smax get NaN, as attention_kernel.
 // One key's score for a query held in registers, before the scale (scores_d64,
 // src/nexterabert.cpp:704-731): the 8 chains a_l = q_l k_l, fma(q[8c+l], k[8c+l], a_l) for
 // c = 1..7, then the HADD tree for a key of a whole group of 8, hsum256's for a tail key.
@@ -950,363 +1405,22 @@ __device__ __forceinline__ float score_d64(const float (&qv)[64], const float * 
                    : ((a[0] + a[4]) + (a[2] + a[6])) + ((a[1] + a[5]) + (a[3] + a[7]));
 }
 
-// Chain-parallel scores: lane L of an 8-lane group computes chain L of one
-// key's dot products with all 16 pairs of the workgroup, a_L = q[L] k[L], then fma(q[8c+L],
-// k[8c+L], a_L) for c = 1..7, and the group adds the 8 chains in the tree
-// ((a0 + a1) + (a2 + a3)) + ((a4 + a5) + (a6 + a7)) by three exchange steps: DPP quad_perm
-// with lane L ^ 1, quad_perm with lane L ^ 2, row_half_mirror with lane 7 - L (the other
-// half of the group). Register i of lane L holds pair i ^ att_chain_g(L): with that
-// assignment every exchange adds the same pair's partial sums from registers of one index
-// (step 1: register i + 8 of the partner to register i, i < 8; step 2: i + 4 to i, i < 4;
-// step 3: i + 2 to i, i < 2), and lane L ends with the scores of pairs att_chain_g(L) and
-// att_chain_g(L) + 1. Each addition is commutative, so the lane order inside a step does not
-// change the bits.
-__device__ __forceinline__ int att_chain_g(int L) { return ((L & 1) ? 8 : 0) ^ ((L & 2) ? 4 : 0) ^ ((L & 4) ? 14 : 0); }
-
-// The tree of the 16 pairs' chain-L values a[i] (pair i ^ att_chain_g(L)) into the two
-// scores of this lane's pairs. The s_nop gives each step's DPP reads their two wait states
-// after the VALU writes of their sources.
-__device__ __forceinline__ void att_chain_tree(const float (&a)[16], float (&s)[2]) {
-    float b[8], c[4];
-    asm("s_nop 1\n\t"
-        "v_add_f32_dpp %0, %16, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %1, %17, %9 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %18, %10 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %3, %19, %11 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %4, %20, %12 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %5, %21, %13 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %6, %22, %14 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %7, %23, %15 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
-        : "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3]), "=&v"(b[4]), "=&v"(b[5]), "=&v"(b[6]), "=&v"(b[7])
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
-          "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]), "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]));
-    asm("s_nop 1\n\t"
-        "v_add_f32_dpp %0, %8, %4 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %1, %9, %5 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %10, %6 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %3, %11, %7 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
-        : "=&v"(c[0]), "=&v"(c[1]), "=&v"(c[2]), "=&v"(c[3])
-        : "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]));
-    asm("s_nop 1\n\t"
-        "v_add_f32_dpp %0, %4, %2 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %1, %5, %3 row_half_mirror row_mask:0xf bank_mask:0xf"
-        : "=&v"(s[0]), "=&v"(s[1])
-        : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]));
-}
-
-// The same for 8 pairs (register i: pair i ^ att_chain_g8(L)): steps of 4, 2 and 1 registers,
-// lane L ending with the score of pair att_chain_g8(L) (0..7, one per lane of the group).
-__device__ __forceinline__ int att_chain_g8(int L) { return ((L & 1) ? 4 : 0) ^ ((L & 2) ? 2 : 0) ^ ((L & 4) ? 7 : 0); }
-__device__ __forceinline__ void att_chain_tree(const float (&a)[8], float (&s)[1]) {
-    float b[4], c[2];
-    asm("s_nop 1\n\t"
-        "v_add_f32_dpp %0, %8, %4 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %1, %9, %5 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %10, %6 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %3, %11, %7 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
-        : "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3])
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]));
-    asm("s_nop 1\n\t"
-        "v_add_f32_dpp %0, %4, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %1, %5, %3 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
-        : "=&v"(c[0]), "=&v"(c[1])
-        : "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
-    asm("s_nop 1\n\t"
-        "v_add_f32_dpp %0, %2, %1 row_half_mirror row_mask:0xf bank_mask:0xf"
-        : "=&v"(s[0])
-        : "v"(c[0]), "v"(c[1]));
-}
-
-__device__ __forceinline__ bool finite4(const v4f & x) {
-    return __builtin_isfinite(x.x) && __builtin_isfinite(x.y) && __builtin_isfinite(x.z) && __builtin_isfinite(x.w);
-}
-#ifndef NXG_ATT_WIDE
-#define NXG_ATT_WIDE 1         // 16 pairs per lane group where LDS allows two workgroups per CU (0: always 8)
-#endif
-constexpr int ATT_P = 16;      // (query, head) pairs per workgroup
-constexpr int ATT_KT = 32;     // keys per staged tile
+constexpr int ATT_KT = 32;     // keys per staged tile of attention_long_kernel
 constexpr int ATT_KS = 68;     // floats per staged row
 
-template <bool WIDE>
-__global__ __launch_bounds__(256) void attention_tile_kernel(attn_params p, int smax) {
-    extern __shared__ __attribute__((aligned(16))) float att_lds[];
-    float * S = att_lds;                                   // [ATT_P][smax]
-    float * tile = att_lds + (size_t) ATT_P * smax;        // [ATT_KT][ATT_KS]
-    __shared__ int lo_s[ATT_P], hi_s[ATT_P];
-    __shared__ float scale_s[ATT_P], inv_s[ATT_P];
-    const int tid = (int) threadIdx.x;
-    const int rep = p.H / p.G, nq = ATT_P / rep;
-    const int n_qblk = (p.T + nq - 1) / nq;
-    const int g = (int) blockIdx.x / n_qblk, t0 = ((int) blockIdx.x - g * n_qblk) * nq;
-
-    if (tid < ATT_P) {
-        const int t = t0 + tid / rep;
-        int lo = 0, hi = 0;
-        float sc = 0.0f;
-        if (t < p.T) {
-            const doc_rows dr = doc_of(p.cu, p.n_seqs, t, p.T);
-            lo = dr.lo;
-            hi = dr.hi;
-            if (p.half >= 0) {
-                lo = max(lo, t - p.half);
-                hi = min(hi, t + p.half + 1);
-            }
-            sc = p.scale[dr.d];
-        }
-        lo_s[tid] = lo;
-        hi_s[tid] = hi;
-        scale_s[tid] = sc;
-    }
-    __syncthreads();
-    // keys any pair reads: [kl, kh)
-    int kl = INT_MAX, kh = INT_MIN;
-#pragma unroll
-    for (int i = 0; i < ATT_P; ++i) {
-        if (hi_s[i] > lo_s[i] && hi_s[i] - lo_s[i] <= smax) {
-            kl = min(kl, lo_s[i]);
-            kh = max(kh, hi_s[i]);
-        }
-    }
-    const float * kg = p.k + (size_t) g * p.T * 64;
-    const float * vg = p.v + (size_t) g * p.T * 64;
-
-    // softmax threads: 16 per pair, pair sp
-    const int sp = tid >> 4, sk = tid & 15;
-    const int n_p = hi_s[sp] - lo_s[sp];
-    const bool valid = n_p > 0 && n_p <= smax;
-    float * Sp = S + (size_t) sp * smax;
-    // staged rows: thread tid moves row (tid >> 4) + 16 r, floats 4 (tid & 15) .. + 3, r < 2;
-    // the next tile's rows are fetched into registers while the current one is used
-    const int st_r = tid >> 4, st_c = 4 * (tid & 15);
-    v4f pre[2];
-    auto fetch = [&](const float * src, int j0) {
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const int j = j0 + st_r + 16 * r;
-            pre[r] = j < kh ? *reinterpret_cast<const v4f *>(src + (size_t) j * 64 + st_c) : v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
-        }
-    };
-    auto stage = [&]() {
-#pragma unroll
-        for (int r = 0; r < 2; ++r) *reinterpret_cast<v4f *>(tile + (st_r + 16 * r) * ATT_KS + st_c) = pre[r];
-    };
-
-    // scores, chain-parallel (att_chain_tree): lane L of an 8-lane group holds element 8c + L
-    // of NPG pairs' queries and computes chain L of one key's dot products with them, so that
-    // each key's 8 values read from LDS serve NPG pairs' FMAs. WIDE: one group per key for all
-    // 16 pairs (128 query registers; for launches whose LDS admits at most two workgroups per
-    // CU); else two groups per key, 8 pairs each (64 registers), each group taking two keys per
-    // tile. Keys are staged chain-major (row j: [L][c], element 8c + L at 8L + c), the queries
-    // likewise through the tile before the first key tile. The scores of keys of whole groups
-    // of 8 come out of the tree; a pair's last n % 8 keys take hsum256's tree, one thread per
-    // (pair, key) afterwards.
-    {
-        constexpr int NPG = WIDE ? ATT_P : ATT_P / 2;          // pairs per 8-lane group
-        constexpr int NO = WIDE ? 2 : 1;                       // scores per lane out of the tree
-        constexpr int NK = WIDE ? 1 : 2;                       // keys per group per tile
-        const int L = tid & 7, gi = tid >> 3;
-        const int gL = WIDE ? att_chain_g(L) : att_chain_g8(L);
-        const int pbase = WIDE ? 0 : NPG * (gi & 1);
-        const int js0 = WIDE ? gi : gi >> 1;
-        {
-            const int pp = tid >> 4, m = tid & 15;
-            const int t = t0 + pp / rep, h = g * rep + pp % rep;
-            const v4f f = *reinterpret_cast<const v4f *>(p.q + (size_t) min(t, p.T - 1) * p.H * 64 + (size_t) h * 64 + 4 * m);
-            const float fe[4] = { f.x, f.y, f.z, f.w };
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int d = 4 * m + u;
-                tile[pp * ATT_KS + (d & 7) * 8 + (d >> 3)] = fe[u];
-            }
-        }
-        __syncthreads();
-        float qr[NPG][8];
-#pragma unroll
-        for (int i = 0; i < NPG; ++i) {
-            const float * src = tile + (pbase + (i ^ gL)) * ATT_KS + L * 8;
-            const v4f a0 = *reinterpret_cast<const v4f *>(src), a1 = *reinterpret_cast<const v4f *>(src + 4);
-            qr[i][0] = a0.x; qr[i][1] = a0.y; qr[i][2] = a0.z; qr[i][3] = a0.w;
-            qr[i][4] = a1.x; qr[i][5] = a1.y; qr[i][6] = a1.z; qr[i][7] = a1.w;
-        }
-        int lo2[NO], ng2[NO], pp2[NO];
-        bool ok2[NO];
-        float sc2[NO];
-#pragma unroll
-        for (int u = 0; u < NO; ++u) {
-            const int pp = pbase + gL + u, n = hi_s[pp] - lo_s[pp];
-            pp2[u] = pp;
-            lo2[u] = lo_s[pp];
-            ok2[u] = n > 0 && n <= smax;
-            ng2[u] = n & ~7;
-            sc2[u] = scale_s[pp];
-        }
-        auto stage_chain = [&]() {
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                float * row = tile + (st_r + 16 * r) * ATT_KS;
-                const float e[4] = { pre[r].x, pre[r].y, pre[r].z, pre[r].w };
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int d = st_c + u;
-                    row[(d & 7) * 8 + (d >> 3)] = e[u];
-                }
-            }
-        };
-        if (kl < kh) fetch(kg, kl);
-        for (int j0 = kl; j0 < kh; j0 += ATT_KT) {
-            __syncthreads();                               // the previous tile (or the queries) read
-            stage_chain();
-            __syncthreads();
-            if (j0 + ATT_KT < kh) fetch(kg, j0 + ATT_KT);
-#pragma unroll
-            for (int r = 0; r < NK; ++r) {
-                const int js = js0 + 16 * r;
-                const float * kp = tile + js * ATT_KS + L * 8;
-                const v4f k0 = *reinterpret_cast<const v4f *>(kp), k1 = *reinterpret_cast<const v4f *>(kp + 4);
-                const float kk[8] = { k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w };
-                float a[NPG];
-#pragma unroll
-                for (int i = 0; i < NPG; ++i) a[i] = qr[i][0] * kk[0];
-#pragma unroll
-                for (int c = 1; c < 8; ++c)
-#pragma unroll
-                    for (int i = 0; i < NPG; ++i) a[i] = __builtin_fmaf(qr[i][c], kk[c], a[i]);
-                float s2[NO];
-                att_chain_tree(a, s2);
-#pragma unroll
-                for (int u = 0; u < NO; ++u) {
-                    const int jr = j0 + js - lo2[u];
-                    if (ok2[u] && jr >= 0 && jr < ng2[u]) S[(size_t) pp2[u] * smax + jr] = s2[u] * sc2[u];
-                }
-            }
-        }
-        if (valid && sk < n_p - (n_p & ~7)) {
-            const int jr = (n_p & ~7) + sk;
-            float qv[64];
-            const int t = t0 + sp / rep, h = g * rep + sp % rep;
-            const float * qrow = p.q + (size_t) min(t, p.T - 1) * p.H * 64 + (size_t) h * 64;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const v4f f = *reinterpret_cast<const v4f *>(qrow + 4 * i);
-                qv[4 * i] = f.x; qv[4 * i + 1] = f.y; qv[4 * i + 2] = f.z; qv[4 * i + 3] = f.w;
-            }
-            Sp[jr] = score_d64(qv, kg + (size_t) (lo_s[sp] + jr) * 64, false) * scale_s[sp];
-        }
-    }
-    __syncthreads();
-
-    // softmax: 16 threads per pair
-    if (valid) softmax_max_exp(Sp, n_p, sk);
-    __syncthreads();
-    {
-        const float inv = softmax_inv(Sp, n_p, sk, valid);
-        if (valid && sk == 0) inv_s[sp] = inv;
-    }
-    __syncthreads();
-    if (valid) softmax_weights(Sp, n_p, sk, inv_s[sp]);
-
-    // values: thread (dim d, pairs 4 pg .. 4 pg + 3); pg is the wave's, so the pairs' key
-    // ranges are scalars and a key outside a pair's range costs a scalar branch
-    const int d = tid & 63, pg = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int vlo[4], vn[4];
-    float acc[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int pp = 4 * pg + i;
-        vlo[i] = __builtin_amdgcn_readfirstlane(lo_s[pp]);
-        vn[i] = __builtin_amdgcn_readfirstlane(hi_s[pp] - lo_s[pp]);
-        if (vn[i] > smax) vn[i] = 0;
-        acc[i] = 0.0f;
-    }
-    // a staged value tile holding a non-finite value (by tile parity): without one, every tile,
-    // also one only partly in a pair's keys, takes the broadcast path, its keys outside the pair's
-    // range adding fma(0, v, acc) = acc (acc is never -0: it starts at +0): banded attention
-    // over 8 x 1,024 tokens 343 -> 291 us, documents of 300 / 45 / 700 tokens 217 -> 144 us
-    __shared__ int vbad_s[2];
-    if (tid < 2) vbad_s[tid] = 0;
-    int par = 0;
-    if (kl < kh) fetch(vg, kl);
-    for (int j0 = kl; j0 < kh; j0 += ATT_KT, par ^= 1) {
-        __syncthreads();                                   // weights written / previous tile read
-        if (tid == 0) vbad_s[par ^ 1] = 0;                 // the previous tile's flag, read by all
-        stage();
-        if (!(finite4(pre[0]) && finite4(pre[1]))) vbad_s[par] = 1;
-        __syncthreads();
-        if (j0 + ATT_KT < kh) fetch(vg, j0 + ATT_KT);
-        const int jn = min(ATT_KT, kh - j0);
-        int a[4], b[4];
-        const bool full = vbad_s[par] == 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {                      // keys [a, b) of the tile are pair i's
-            a[i] = min(max(vlo[i] - j0, 0), jn);
-            b[i] = max(min(vlo[i] + vn[i] - j0, jn), a[i]);
-        }
-        // the tile's weights: pair i's weight of key j0 + l in lane l (l < 32), read once and
-        // broadcast per key (readlane), so the key loop reads only the value row from LDS
-        // weights of keys j0 + k (w0) and j0 + 16 + k (w1) of pair i in lane k of every 16-lane row
-        float w0[4], w1[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int jr = j0 + (d & 15) - vlo[i];
-            w0[i] = (jr >= 0 && jr < vn[i]) ? S[(size_t) (4 * pg + i) * smax + jr] : 0.0f;
-            w1[i] = (jr + 16 >= 0 && jr + 16 < vn[i]) ? S[(size_t) (4 * pg + i) * smax + jr + 16] : 0.0f;
-        }
-        auto wk = [&](int i, int jj) {
-            return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(jj < 16 ? w0[i] : w1[i]), jj & 15));
-        };
-        if (full) {
-            float vt[ATT_KT];                              // the tile's values of dimension d, read up front
-#pragma unroll
-            for (int jj = 0; jj < ATT_KT; ++jj) vt[jj] = tile[jj * ATT_KS + d];
-            fmac_bcast4_16(acc, w0, vt);
-            fmac_bcast4_16(acc, w1, vt + 16);
-        } else {
-            for (int jj = 0; jj < jn; ++jj) {
-                const float v = tile[jj * ATT_KS + d];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (jj >= a[i] && jj < b[i]) acc[i] = __builtin_fmaf(wk(i, jj), v, acc[i]);
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int pp = 4 * pg + i, t = t0 + pp / rep, h = g * rep + pp % rep;
-        if (t >= p.T) continue;
-        const int n = hi_s[pp] - lo_s[pp];
-        p.out[(size_t) t * p.H * 64 + (size_t) h * 64 + d] = (n > 0 && n <= smax) ? acc[i] : __uint_as_float(0x7fc00000u);
-    }
-}
-
-
-// attention_tile_kernel's pairs, thread mapping and per-pair order for documents whose
-// scores do not fit in LDS: nothing is kept per key; the scores are computed three times,
-// bit-identically.
+// The same pairs for documents whose scores fit neither LDS nor a workspace: nothing is kept per
+// key; the scores are computed three times, bit-identically, on the vector unit.
 //   pass 1  the maximum (a NaN first score wins, else the largest score that is not NaN)
 //   pass 2  e = exp256(s - m) (grouped keys) or the C library's expf (the n % 8 tail keys);
 //           each tile's e go through LDS so that lanes l < 8 of a pair add keys 8i + l in
 //           order of i, as softmax_exp's 8 accumulator lanes do; the tail e are kept apart and
 //           added after hsum256, in order
 //   pass 3  w = e * (1 / sum) per key through LDS, then thread (dim d, 4 pairs) acc = fma(w,
-//           v[d], acc) over the keys in order, as attention_tile_kernel (the tile's weights
-//           read once per lane and broadcast per key by DPP row_newbcast, or by readlane with a
-//           per-key range test on partial tiles (ZW: only on tiles with an Inf or NaN value))
+//           v[d], acc) over the keys in order: a tile's weights are read once per lane and
+//           broadcast per key by DPP row_newbcast (keys outside a pair's range with weight 0), or
+//           by readlane with a per-key range test on tiles with an Inf or NaN value
 // Keys and values are staged ATT_KT at a time ([key][ATT_KS]).
-// STORED: pass 1 also writes each score to the workgroup's slot of the workspace sc
-// ([gridDim.x][ATT_P][max_keys] floats, pair-relative key index), and passes 2 and 3 read the
-// scores back instead of recomputing them, the same bits; pass 2 then needs no staged keys
-// (lane l < 8 of a pair adds keys 16b + l and 16b + 8 + l, the second taken from lane l + 8),
-// pass 3 stages only the values. ESTORE: pass 2 also writes each e = exp(s - m) over
-// its score and pass 3 takes w = e * (1 / sum) from it (the same bits as recomputing e).
-// One call is the tile bt = (KV head, query block).
-#ifndef NXG_ATT_STORED_WIDE
-#define NXG_ATT_STORED_WIDE 0  // attention_stored_kernel's scores: 16 pairs per lane group (0: 8)
-#endif
-#ifndef NXG_ATT_E_STORE_MIB
-#define NXG_ATT_E_STORE_MIB 192   // the largest workspace in use (all slots) for which pass 2 stores e
-#endif
-template <bool STORED, bool ESTORE, bool ZW>
-__device__ __forceinline__ void attention_long_tile(const attn_params & p, float * __restrict__ sc, int bt) {
+__global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
     __shared__ __attribute__((aligned(16))) float tile[ATT_KT * ATT_KS];
     __shared__ float E[ATT_P][ATT_KT + 1];                 // one tile's e (pass 2) or w (pass 3)
     __shared__ float tail_e[ATT_P][8];
@@ -1315,7 +1429,7 @@ __device__ __forceinline__ void attention_long_tile(const attn_params & p, float
     const int tid = (int) threadIdx.x;
     const int rep = p.H / p.G, nq = ATT_P / rep;
     const int n_qblk = (p.T + nq - 1) / nq;
-    const int g = bt / n_qblk, t0 = (bt - g * n_qblk) * nq;
+    const int g = (int) blockIdx.x / n_qblk, t0 = ((int) blockIdx.x - g * n_qblk) * nq;
 
     if (tid < ATT_P) {
         const int t = t0 + tid / rep;
@@ -1350,16 +1464,13 @@ __device__ __forceinline__ void attention_long_tile(const attn_params & p, float
     const int sp = tid >> 4, sk = tid & 15;
     const int plo = lo_s[sp], n_p = hi_s[sp] - plo, ng_p = n_p & ~7;
     const bool valid = n_p > 0 && n_p <= p.max_keys;     // more keys than max_keys: NaN, as the other kernels
-    float * const scp = STORED ? sc + ((size_t) blockIdx.x * ATT_P + sp) * (size_t) p.max_keys : nullptr;
-    // this thread's pair's query (STORED: only for its tail keys, loaded there)
+    // this thread's pair's query
     float qv[64];
     const float * const qrow = p.q + (size_t) min(t0 + sp / rep, p.T - 1) * p.H * 64 + (size_t) (g * rep + sp % rep) * 64;
-    if constexpr (!STORED) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const v4f f = *reinterpret_cast<const v4f *>(qrow + 4 * i);
-            qv[4 * i] = f.x; qv[4 * i + 1] = f.y; qv[4 * i + 2] = f.z; qv[4 * i + 3] = f.w;
-        }
+    for (int i = 0; i < 16; ++i) {
+        const v4f f = *reinterpret_cast<const v4f *>(qrow + 4 * i);
+        qv[4 * i] = f.x; qv[4 * i + 1] = f.y; qv[4 * i + 2] = f.z; qv[4 * i + 3] = f.w;
     }
     const float scale = scale_s[sp];
     const int st_r = tid >> 4, st_c = 4 * (tid & 15);
@@ -1377,122 +1488,7 @@ __device__ __forceinline__ void attention_long_tile(const attn_params & p, float
     };
 
     // pass 1: the maximum
-    if constexpr (STORED) {
-        // the scores chain-parallel, as attention_tile_kernel (att_chain_tree; SW: 16 pairs
-        // per lane group, else 8 pairs and two keys per group and tile), each written to the
-        // workspace; the maxima of a pair's key slots meet in E, then its 16 lanes; a pair's
-        // last n % 8 keys by hsum256's tree, one thread per key
-        constexpr bool SW = NXG_ATT_STORED_WIDE;
-        constexpr int NPG = SW ? ATT_P : ATT_P / 2;            // pairs per 8-lane group
-        constexpr int NO = SW ? 2 : 1;                         // scores per lane out of the tree
-        constexpr int NK = SW ? 1 : 2;                         // keys per group per tile
-        const int L = tid & 7, gi = tid >> 3;
-        const int gL = SW ? att_chain_g(L) : att_chain_g8(L);
-        const int pbase = SW ? 0 : NPG * (gi & 1);
-        const int js0 = SW ? gi : gi >> 1;
-        {
-            const int pp = tid >> 4, m = tid & 15;
-            const int t = t0 + pp / rep, h = g * rep + pp % rep;
-            const v4f f = *reinterpret_cast<const v4f *>(p.q + (size_t) min(t, p.T - 1) * p.H * 64 + (size_t) h * 64 + 4 * m);
-            const float fe[4] = { f.x, f.y, f.z, f.w };
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int d = 4 * m + u;
-                tile[pp * ATT_KS + (d & 7) * 8 + (d >> 3)] = fe[u];
-            }
-        }
-        __syncthreads();
-        float qr[NPG][8];
-#pragma unroll
-        for (int i = 0; i < NPG; ++i) {
-            const float * src = tile + (pbase + (i ^ gL)) * ATT_KS + L * 8;
-            const v4f a0 = *reinterpret_cast<const v4f *>(src), a1 = *reinterpret_cast<const v4f *>(src + 4);
-            qr[i][0] = a0.x; qr[i][1] = a0.y; qr[i][2] = a0.z; qr[i][3] = a0.w;
-            qr[i][4] = a1.x; qr[i][5] = a1.y; qr[i][6] = a1.z; qr[i][7] = a1.w;
-        }
-        int lo2[NO], ng2[NO];
-        bool ok2[NO];
-        float sc2[NO], mx2[NO];
-        float * sp2[NO];
-#pragma unroll
-        for (int u = 0; u < NO; ++u) {
-            const int pp = pbase + gL + u, n = hi_s[pp] - lo_s[pp];
-            lo2[u] = lo_s[pp];
-            ok2[u] = n > 0 && n <= p.max_keys;
-            ng2[u] = n & ~7;
-            sc2[u] = scale_s[pp];
-            mx2[u] = -__builtin_inff();
-            sp2[u] = sc + ((size_t) blockIdx.x * ATT_P + pp) * (size_t) p.max_keys;
-        }
-        auto stage_chain = [&]() {
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                float * row = tile + (st_r + 16 * r) * ATT_KS;
-                const float e[4] = { pre[r].x, pre[r].y, pre[r].z, pre[r].w };
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int d = st_c + u;
-                    row[(d & 7) * 8 + (d >> 3)] = e[u];
-                }
-            }
-        };
-        if (kl < kh) fetch(kg, kl);
-        for (int j0 = kl; j0 < kh; j0 += ATT_KT) {
-            __syncthreads();                               // the previous tile (or the queries) read
-            stage_chain();
-            __syncthreads();
-            if (j0 + ATT_KT < kh) fetch(kg, j0 + ATT_KT);
-#pragma unroll
-            for (int r = 0; r < NK; ++r) {
-                const int js = js0 + 16 * r;
-                const float * kp = tile + js * ATT_KS + L * 8;
-                const v4f k0 = *reinterpret_cast<const v4f *>(kp), k1 = *reinterpret_cast<const v4f *>(kp + 4);
-                const float kk[8] = { k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w };
-                float a[NPG];
-#pragma unroll
-                for (int i = 0; i < NPG; ++i) a[i] = qr[i][0] * kk[0];
-#pragma unroll
-                for (int c = 1; c < 8; ++c)
-#pragma unroll
-                    for (int i = 0; i < NPG; ++i) a[i] = __builtin_fmaf(qr[i][c], kk[c], a[i]);
-                float s2[NO];
-                att_chain_tree(a, s2);
-#pragma unroll
-                for (int u = 0; u < NO; ++u) {
-                    const int jr = j0 + js - lo2[u];
-                    if (ok2[u] && jr >= 0 && jr < ng2[u]) {
-                        const float s = s2[u] * sc2[u];
-                        mx2[u] = fmaxf(mx2[u], s);
-                        sp2[u][jr] = s;
-                        if (jr == 0) s0_s[pbase + gL + u] = s;
-                    }
-                }
-            }
-        }
-        // SW: pair gL + u's maxima over key slots js0 (0..31); else pair pbase + gL's over
-        // key slots js0 and js0 + 16 in slot js0 (0..15)
-#pragma unroll
-        for (int u = 0; u < NO; ++u) E[pbase + gL + u][js0] = mx2[u];
-        __syncthreads();
-        float mx = SW ? fmaxf(E[sp][sk], E[sp][sk + 16]) : E[sp][sk];
-        if (valid && sk < n_p - ng_p) {
-            const int jr = ng_p + sk;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const v4f f = *reinterpret_cast<const v4f *>(qrow + 4 * i);
-                qv[4 * i] = f.x; qv[4 * i + 1] = f.y; qv[4 * i + 2] = f.z; qv[4 * i + 3] = f.w;
-            }
-            const float s = score_d64(qv, kg + (size_t) (plo + jr) * 64, false) * scale;
-            mx = fmaxf(mx, s);
-            scp[jr] = s;
-            if (jr == 0) s0_s[sp] = s;
-        }
-#pragma unroll
-        for (int sft = 8; sft >= 1; sft >>= 1) mx = fmaxf(mx, __shfl_xor(mx, sft));
-        __syncthreads();                                   // s0_s written
-        if (valid && sk == 0) m_s[sp] = __builtin_isnan(s0_s[sp]) ? s0_s[sp] : mx;
-        __syncthreads();
-    } else {
+    {
         float mx = -__builtin_inff();
         if (kl < kh) fetch(kg, kl);
         for (int j0 = kl; j0 < kh; j0 += ATT_KT) {
@@ -1507,7 +1503,6 @@ __device__ __forceinline__ void attention_long_tile(const attn_params & p, float
                 const float s = score_d64(qv, tile + (sk + 16 * r) * ATT_KS, jr < ng_p) * scale;
                 mx = fmaxf(mx, s);
                 if (jr == 0) s0_s[sp] = s;
-                if constexpr (STORED) scp[jr] = s;
             }
         }
 #pragma unroll
@@ -1519,50 +1514,7 @@ __device__ __forceinline__ void attention_long_tile(const attn_params & p, float
     const float m = m_s[sp];
 
     // pass 2: the ordered sum of the exponentials
-    if constexpr (STORED) {
-        float ls = 0.0f;
-        const int ng = valid ? ng_p : 0;                   // the same for the 16 lanes of a pair
-        constexpr int U = 16;                              // 16-key steps per batch of loads
-        float cur[U], nxt[U];
-        auto load = [&](float (&dst)[U], int b) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int jr = b + 16 * u + sk;
-                dst[u] = jr < ng ? scp[jr] : 0.0f;
-            }
-        };
-        if (ng > 0) load(cur, 0);
-        for (int b = 0; b < ng; b += 16 * U) {
-            if (b + 16 * U < ng) load(nxt, b + 16 * U);    // the next batch in flight meanwhile
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (b + 16 * u >= ng) break;               // uniform over the pair's 16 lanes
-                const int jr = b + 16 * u + sk;
-                const float e = jr < ng ? exp_cephes(cur[u] - m) : 0.0f;
-                if (ESTORE && jr < ng) scp[jr] = e;        // pass 3 reads e in place of the score
-                const float e8 = __shfl_down(e, 8, 16);    // key jr + 8, from lane sk + 8
-                if (sk < 8) {
-                    ls = ls + e;
-                    if (jr + 8 < ng) ls = ls + e8;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) cur[u] = nxt[u];
-        }
-        ls = ls + __shfl_xor(ls, 4);                       // lanes 8..15 hold 0 and stay among themselves
-        ls = ls + __shfl_xor(ls, 2);
-        ls = ls + __shfl_xor(ls, 1);
-        if (valid && sk == 0) {
-            float sum = ls;
-            for (int jr = ng_p; jr < n_p; ++jr) {
-                const float e = expf_libm(scp[jr] - m);
-                if (ESTORE) scp[jr] = e;
-                sum = sum + e;
-            }
-            inv_s[sp] = 1.0f / sum;
-        }
-        __syncthreads();
-    } else {
+    {
         float ls = 0.0f;
         if (kl < kh) fetch(kg, kl);
         for (int j0 = kl; j0 < kh; j0 += ATT_KT) {
@@ -1613,74 +1565,42 @@ __device__ __forceinline__ void attention_long_tile(const attn_params & p, float
         vn[i] = __builtin_amdgcn_readfirstlane(n <= p.max_keys ? n : 0);
         acc[i] = 0.0f;
     }
-    float snx[2] = { 0.0f, 0.0f };                          // STORED: the next tile's scores of this thread
-    auto sfetch = [&](int j0) {
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const int jr = j0 + sk + 16 * r - plo;
-            snx[r] = valid && jr >= 0 && jr < n_p ? scp[jr] : 0.0f;
-        }
-    };
-    // ZW: a staged value tile holding a non-finite value (by tile parity), as attention_tile_kernel:
-    // without one, a partial tile takes the broadcast path with zero weights outside a pair's keys
+    // a staged value tile holding a non-finite value (by tile parity): without one, a partial tile
+    // takes the broadcast path with zero weights outside a pair's keys
     __shared__ int vbad_s[2];
     if (tid < 2) vbad_s[tid] = 0;
     int par = 0;
-    if (kl < kh) {
-        fetch(STORED ? vg : kg, kl);
-        if constexpr (STORED) sfetch(kl);
-    }
+    if (kl < kh) fetch(kg, kl);
     for (int j0 = kl; j0 < kh; j0 += ATT_KT, par ^= 1) {
         __syncthreads();                                   // E and the tile are free
-        if (ZW && tid == 0) vbad_s[par ^ 1] = 0;           // the previous tile's flag, read by all
+        if (tid == 0) vbad_s[par ^ 1] = 0;                 // the previous tile's flag, read by all
         stage();
-        if constexpr (STORED) {
-            if (ZW && !(finite4(pre[0]) && finite4(pre[1]))) vbad_s[par] = 1;
+        __syncthreads();
+        fetch(vg, j0);                                     // this tile's values, staged after the weights
 #pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const int kt = sk + 16 * r, jr = j0 + kt - plo;
-                if (!valid || jr < 0 || jr >= n_p) {
-                    if (ZW) E[sp][kt] = 0.0f;
-                    continue;
-                }
-                const float s = snx[r];
-                if (ESTORE) E[sp][kt] = s * inv;          // s holds e = exp(score - m), written by pass 2
-                else E[sp][kt] = (jr < ng_p ? exp_cephes(s - m) : expf_libm(s - m)) * inv;
+        for (int r = 0; r < 2; ++r) {
+            const int kt = sk + 16 * r, jr = j0 + kt - plo;
+            if (!valid || jr < 0 || jr >= n_p) {
+                E[sp][kt] = 0.0f;
+                continue;
             }
-            __syncthreads();                               // the values and the weights are in LDS
-            if (j0 + ATT_KT < kh) {
-                fetch(vg, j0 + ATT_KT);
-                sfetch(j0 + ATT_KT);
-            }
-        } else {
-            __syncthreads();
-            fetch(vg, j0);                                 // this tile's values, staged after the weights
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const int kt = sk + 16 * r, jr = j0 + kt - plo;
-                if (!valid || jr < 0 || jr >= n_p) {
-                    if (ZW) E[sp][kt] = 0.0f;
-                    continue;
-                }
-                const float s = score_d64(qv, tile + kt * ATT_KS, jr < ng_p) * scale;
-                E[sp][kt] = (jr < ng_p ? exp_cephes(s - m) : expf_libm(s - m)) * inv;
-            }
-            __syncthreads();                               // the keys have been read
-            stage();
-            if (ZW && !(finite4(pre[0]) && finite4(pre[1]))) vbad_s[par] = 1;
-            __syncthreads();
-            if (j0 + ATT_KT < kh) fetch(kg, j0 + ATT_KT);
+            const float s = score_d64(qv, tile + kt * ATT_KS, jr < ng_p) * scale;
+            E[sp][kt] = (jr < ng_p ? exp_cephes(s - m) : expf_libm(s - m)) * inv;
         }
+        __syncthreads();                                   // the keys have been read
+        stage();
+        if (!(finite4(pre[0]) && finite4(pre[1]))) vbad_s[par] = 1;
+        __syncthreads();
+        if (j0 + ATT_KT < kh) fetch(kg, j0 + ATT_KT);
         const int jn = min(ATT_KT, kh - j0);
         // pair i's weights of the tile: lane l holds key j0 + l (l < 32), broadcast per key
         int a[4], b[4];
-        bool full = ZW ? vbad_s[par] == 0 : jn == ATT_KT;
+        const bool full = vbad_s[par] == 0;
         float w0[4], w1[4];                                // keys j0 + k, j0 + 16 + k in lane k of each row
 #pragma unroll
         for (int i = 0; i < 4; ++i) {                      // keys [a, b) of the tile are pair i's
             a[i] = min(max(vlo[i] - j0, 0), jn);
             b[i] = max(min(vlo[i] + vn[i] - j0, jn), a[i]);
-            if (!ZW) full = full && a[i] == 0 && b[i] == jn;
             w0[i] = E[4 * pg + i][d & 15];
             w1[i] = E[4 * pg + i][16 + (d & 15)];
         }
@@ -1708,31 +1628,6 @@ __device__ __forceinline__ void attention_long_tile(const attn_params & p, float
         if (t >= p.T) continue;
         const int n = hi_s[pp] - lo_s[pp];
         p.out[(size_t) t * p.H * 64 + (size_t) h * 64 + d] = (n > 0 && n <= p.max_keys) ? acc[i] : __uint_as_float(0x7fc00000u);
-    }
-}
-
-__global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
-    attention_long_tile<false, false, true>(p, nullptr, (int) blockIdx.x);
-}
-
-// The scores kept in the workspace: a persistent grid, one slot of sc per workgroup, which
-// takes tiles blockIdx.x, blockIdx.x + gridDim.x, ... ESTORE: pass 2 stores the exponentials.
-// ZW (banded launches, where most value tiles are partial for some pair): partial tiles on the
-// broadcast path (16,384 keys in bands of 2,601 5.27 -> 5.18 ms); without a band only a pair's
-// last tile is partial, and the flags cost 1-2% (8,192 keys 8.31 -> 8.46 ms).
-// Three workgroups per CU (at most 168 registers; 8 pairs per lane group in pass 1, as 16 would
-// spill): 16,384 keys 40.9 -> 34.7 ms, 8,192 keys 10.2 -> 8.4 ms against two workgroups per CU with
-// 16 pairs per group (256 registers); four per CU (128 registers) spill and lose 1-10%.
-#ifndef NXG_ATT_STORED_MINB
-#define NXG_ATT_STORED_MINB 3
-#endif
-template <bool ESTORE, bool ZW>
-__global__ __launch_bounds__(256, NXG_ATT_STORED_MINB) void attention_stored_kernel(attn_params p, float * __restrict__ sc) {
-    const int nq = ATT_P / (p.H / p.G);
-    const int n_tiles = p.G * ((p.T + nq - 1) / nq);
-    for (int bt = (int) blockIdx.x; bt < n_tiles; bt += (int) gridDim.x) {
-        __syncthreads();                                   // the previous tile's shared reads are done
-        attention_long_tile<true, ESTORE, ZW>(p, sc, bt);
     }
 }
 
@@ -2319,25 +2214,6 @@ __device__ __forceinline__ const int8_t * uniform_ptr(const int8_t * ptr) {
     const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) v);
     const uint32_t hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (v >> 32));
     return reinterpret_cast<const int8_t *>((uintptr_t) (((uint64_t) hi << 32) | lo));
-}
-
-// This lane's number, computed where it is used: an asm the compiler cannot hoist, so
-// that values derived from it are not kept live across a loop (register pressure).
-__device__ __forceinline__ int lane_here() {
-    int l;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-    return l;
-}
-
-// A raw buffer resource over `bytes` bytes at `base` (gfx9 descriptor word 3): buffer
-// loads take a scalar base, a scalar offset and one vector offset, so that a wave's
-// address arithmetic stays on the scalar unit, and they count in vmcnt only.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void * base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short) 0, (int) bytes, 0x00020000);
-}
-// 16 bytes per lane at byte soff (wave-uniform) + voff (per lane) of the buffer.
-__device__ __forceinline__ v4i bload16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, (int) voff, (int) soff, 0);
 }
 
 // dma16 from a scalar base: lane l copies the 16 bytes at base + voff_l to LDS
@@ -3707,10 +3583,10 @@ static int32_t launch_produce(const char * what, const Src & src, int32_t T, int
     return launch_check(what);
 }
 
-// Dynamic LDS the tiled attention kernel may take on the current device: the device's
+// Dynamic LDS the attention kernel may take on the current device: the device's
 // shared memory per workgroup less the kernel's static arrays, with the attribute that
 // allows more than the default raised to it, once per thread and device (as check_device).
-static size_t attention_tile_lds_limit() {
+static size_t attention_lds_limit() {
     static thread_local size_t limit = 0;
     static thread_local int limit_dev = -1;
     int dev = 0;
@@ -3722,16 +3598,16 @@ static size_t attention_tile_lds_limit() {
         int v = 0;
         limit = 0;
         if (dev >= 0 &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 1024) {
-            const size_t want = (size_t) v - 1024;           // static arrays of the kernel: 4 x ATT_P words
-            if (hipFuncSetAttribute((const void *) attention_tile_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > ATT_STATIC_LDS) {
+            const size_t want = (size_t) v - ATT_STATIC_LDS;
+            if (hipFuncSetAttribute((const void *) attention_mfma_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int) want) == hipSuccess &&
-                hipFuncSetAttribute((const void *) attention_tile_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                hipFuncSetAttribute((const void *) attention_mfma_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int) want) == hipSuccess) {
                 limit = want;
             } else {
                 (void) hipGetLastError();
-                limit = 65536 - 1024;
+                limit = 65536 - ATT_STATIC_LDS;
             }
         }
         limit_dev = dev;
@@ -3897,8 +3773,6 @@ int32_t nxg_block_mean_quantize_rows(const float * h, const float * g, const int
                           n_blocks, n_in, act_max, q, sx, stream);
 }
 
-// Resident workgroups of attention_stored_kernel on the device (its persistent grid and
-// the workspace slots), queried once.
 // The scratch of nxg_attention_noalloc: a device array of the code object, so the entry point
 // allocates nothing. Each GPU the library runs on holds its own copy at its own address (until
 // the process ends); host code uses that address, found once per device by
@@ -3927,22 +3801,33 @@ static int scratch_of_device(void ** out) {
     return NXG_OK;
 }
 
-// Workgroups of the long attention kernel resident at once on the current device (its
-// compute units x occupancy), each needing one workspace slot. Cached per thread for the
-// device it was computed on, like check_device's device check.
-static long long attention_long_slots() {
+// Tiles of LDS a workgroup of attention_mfma_kernel<true> takes: those of four workgroups per CU;
+// of two past 4,096 keys, where the slots of four (4 MiB each at 65,536 keys) and the keys and
+// values they read at different times outgrow the caches (2,048 keys 265 us with four, 282 with
+// two; 4,096 keys 1.11 and 1.10 ms; 16,384 keys 26.7 and 26.0 ms; 65,536 keys 543 and 463 ms).
+static int attention_ws_lds_tiles(int need) {
+    const int per_cu = need <= 257 ? 4 : 2;
+    return ((int) ((attention_lds_limit() + ATT_STATIC_LDS) / per_cu - ATT_STATIC_LDS) / ATT_TILE_BYTES) & ~(ATT_VC - 1);
+}
+
+// Workgroups of attention_mfma_kernel<true> resident at once on the current device (its compute
+// units x occupancy), each needing one workspace slot. Cached per thread for the device it was
+// computed on, like check_device's device check.
+static long long attention_slots(int need) {
     static thread_local long long slots = 0;
-    static thread_local int slots_dev = -1;
+    static thread_local int slots_dev = -1, slots_lds = -1;
+    const int lds_tiles = attention_ws_lds_tiles(need);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
         (void) hipGetLastError();
         dev = -1;
     }
-    if (dev < 0 || dev != slots_dev) {
+    if (dev < 0 || dev != slots_dev || lds_tiles != slots_lds) {
         int cus = 0, per_cu = 0;
         if (dev >= 0 &&
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attention_stored_kernel<false, false>, 256, 0) == hipSuccess &&
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attention_mfma_kernel<true>, 256,
+                                                         (size_t) lds_tiles * ATT_TILE_BYTES) == hipSuccess &&
             cus > 0 && per_cu > 0) {
             slots = (long long) cus * per_cu;
         } else {
@@ -3950,42 +3835,41 @@ static long long attention_long_slots() {
             slots = 256;
         }
         slots_dev = dev;
+        slots_lds = lds_tiles;
     }
     return slots;
 }
 
-// The launch nxg_attention_ws makes for (T, heads, max_keys): 0 tile kernel, 1 stored kernel
-// given a workspace slot (else the tile kernel where its LDS fits, else the recomputing long
-// kernel), 2 row kernel; the tiles, the workspace bytes of one slot, and whether the tile
-// kernel's LDS fits.
+// The launch nxg_attention_ws makes for (T, heads, max_keys): 0 the scores in LDS, 1 in LDS and a
+// workspace slot given one (else in LDS where they fit, else the recomputing long kernel), 2 row
+// kernel; the workgroups' tiles, the key tiles of one, the bytes of one slot, and whether all key
+// tiles fit in LDS.
 struct attn_plan {
     int kind;
     long long n_tiles;
+    int need;
     long long slot_bytes;
-    bool tile_fits;
+    bool lds_fits;
 };
 
-// The tile kernel keeps its scores in LDS: ATT_P * smax floats beside one staged tile. Where
-// that leaves room for one workgroup per CU, or for two while the launch has more than two
-// rounds of them, attention_stored_kernel (the scores in a workspace slot, three workgroups
-// per CU) is faster: 2,048 keys 970 -> 560 us, 1,536 keys 560 -> 320 us, 2 x 1,024 keys
-// 314 -> 279 us, 8 x 1,024 keys 1,098 -> 1,015 us; one 1,024-key document (1,024 tiles, two
-// rounds) stays 3% faster on the tile kernel.
-static bool attention_tile_first(size_t tile_lds, size_t lds_max, long long n_tiles) {
-    if (tile_lds > lds_max) return false;
-    const size_t per_cu = (lds_max + 1024) / (tile_lds + 1024);   // the static 1 KiB included
-    return per_cu >= 3 || (per_cu == 2 && n_tiles <= 4LL * device_cus());
-}
-
+// A workgroup's pairs attend to at most max_keys + (its query rows - 1) keys of one document.
+// Where their LDS leaves room for one workgroup per CU, or for two while the launch has more
+// than two rounds of them, the workspace keeps what is past a quarter of a CU's LDS, so that four
+// run: 8 x 1,024 keys 564 -> 516 us, 2,048 keys 357 -> 265 us. Otherwise the scores stay in LDS
+// (512 keys 24.8 us, 25.4 with a workspace).
 static attn_plan plan_attention(int32_t T, int32_t n_head, int32_t n_kv_head, int32_t max_keys) {
     const int rep = n_head / n_kv_head;
-    if (ATT_P % rep != 0) return {2, 0, 0, false};
-    const long long n_tiles = (long long) n_kv_head * ((T + ATT_P / rep - 1) / (ATT_P / rep));
-    const int smax = (max_keys + 3) & ~3;
-    const size_t tile_lds = ((size_t) ATT_P * smax + (size_t) ATT_KT * ATT_KS) * sizeof(float);
-    const size_t lds_max = attention_tile_lds_limit();
-    if (attention_tile_first(tile_lds, lds_max, n_tiles)) return {0, n_tiles, 0, true};
-    return {1, n_tiles, (long long) ATT_P * max_keys * (long long) sizeof(float), tile_lds <= lds_max};
+    if (ATT_P % rep != 0) return {2, 0, 0, 0, false};
+    const int nq = ATT_P / rep;
+    const long long n_tiles = (long long) n_kv_head * ((T + nq - 1) / nq);
+    const long long slot_bytes = (long long) ATT_P * max_keys * (long long) sizeof(float);
+    if (max_keys > ATT_MAX_KEYS) return {1, n_tiles, 0, slot_bytes, false};
+    const int need = (max_keys + nq - 1 + ATT_TILE - 1) / ATT_TILE;
+    const size_t lds = (size_t) need * ATT_TILE_BYTES, lds_max = attention_lds_limit();
+    if (lds > lds_max) return {1, n_tiles, need, slot_bytes, false};
+    const size_t per_cu = (lds_max + ATT_STATIC_LDS) / (lds + ATT_STATIC_LDS);
+    const bool lds_first = per_cu >= 3 || (per_cu == 2 && n_tiles <= 4LL * device_cus());
+    return {lds_first ? 0 : 1, n_tiles, need, slot_bytes, true};
 }
 
 int64_t nxg_attention_workspace_bytes(int32_t T, int32_t n_head, int32_t n_kv_head, int32_t max_keys) {
@@ -3998,7 +3882,7 @@ int64_t nxg_attention_workspace_bytes(int32_t T, int32_t n_head, int32_t n_kv_he
     if (rc) return rc;
     const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
     if (pl.kind != 1) return 0;
-    return std::min(pl.n_tiles, attention_long_slots()) * pl.slot_bytes;
+    return std::min(pl.n_tiles, attention_slots(pl.need)) * pl.slot_bytes;
 }
 
 int32_t nxg_attention_noalloc(const float * q, const float * k, const float * v, const int32_t * cu_offsets,
@@ -4013,13 +3897,13 @@ int32_t nxg_attention_noalloc(const float * q, const float * k, const float * v,
     if (rc) return rc;
     const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
     const bool use_scratch = pl.kind == 1 && pl.slot_bytes <= (long long) NXG_NOALLOC_SCRATCH_BYTES;
-    if (pl.kind == 1 && !use_scratch && !pl.tile_fits) {
+    if (pl.kind == 1 && !use_scratch && !pl.lds_fits) {
         return fail(NXG_EINVAL,
                     "attention_noalloc: max_keys=%d needs %lld bytes per workgroup's scores; the static scratch "
                     "holds %lld (at most %lld keys)", max_keys, pl.slot_bytes, (long long) NXG_NOALLOC_SCRATCH_BYTES,
                     (long long) NXG_NOALLOC_SCRATCH_BYTES / (ATT_P * (long long) sizeof(float)));
     }
-    void * ws = nullptr;                       // none: the tile kernel, its scores in LDS
+    void * ws = nullptr;                       // none: the scores in LDS
     if (use_scratch) {
         rc = scratch_of_device(&ws);
         if (rc) return rc;
@@ -4053,43 +3937,27 @@ int32_t nxg_attention_ws(const float * q, const float * k, const float * v, cons
     int rc = check_device();
     if (rc) return rc;
     attn_params p{q, k, v, cu_offsets, scale, out, n_seqs, T, n_head, n_kv_head, half < 0 ? -1 : half, max_keys};
-    // the tiled kernel when its LDS (scores of ATT_P pairs + one staged tile) fits a workgroup
-    // and attention_tile_first prefers it, or no workspace slot is given
     const int rep = n_head / n_kv_head;
-    const int smax = (max_keys + 3) & ~3;
-    const size_t tile_lds = ((size_t) ATT_P * smax + (size_t) ATT_KT * ATT_KS) * sizeof(float);
-    if (ATT_P % rep == 0) {
-        const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
-        const long long n_tiles = pl.n_tiles;
-        const size_t lds_max = attention_tile_lds_limit();
-        // scores written once into the workspace: as many slots as it holds, up to the resident workgroups
-        const long long n_slots =
-            pl.kind == 1 ? std::min({n_tiles, attention_long_slots(), (long long) (workspace_bytes / pl.slot_bytes)}) : 0;
-        if (tile_lds <= lds_max && n_slots < 1) {
-            // fewer than 3 workgroups per CU by LDS (the static 1 KiB included): 16 pairs per lane group
-            if (NXG_ATT_WIDE && 3 * (tile_lds + 1024) > lds_max + 1024) {
-                attention_tile_kernel<true><<<dim3((unsigned) n_tiles), dim3(256), tile_lds, (hipStream_t) stream>>>(p, smax);
-            } else {
-                attention_tile_kernel<false><<<dim3((unsigned) n_tiles), dim3(256), tile_lds, (hipStream_t) stream>>>(p, smax);
+    const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
+    if (pl.kind != 2) {
+        hipStream_t s = (hipStream_t) stream;
+        if (pl.kind == 1 && pl.need > 0) {
+            // as many slots as the workspace holds, up to the resident workgroups
+            const int lds_tiles = attention_ws_lds_tiles(pl.need), ws_tiles = std::max(pl.need - lds_tiles, 1);
+            const long long n_slots = std::min({pl.n_tiles, attention_slots(pl.need),
+                                                (long long) (workspace_bytes / ((long long) ws_tiles * ATT_TILE_BYTES))});
+            if (n_slots >= 1) {
+                attention_mfma_kernel<true><<<dim3((unsigned) n_slots), dim3(256), (size_t) lds_tiles * ATT_TILE_BYTES, s>>>(
+                    p, lds_tiles, ws_tiles, (float *) workspace);
+                return launch_check("attention_mfma_kernel");
             }
-            return launch_check("attention_tile_kernel");
         }
-        if (n_slots >= 1) {
-            // e stored by pass 2 (4 more bytes per (pair, key)) pays while the slots in use stay
-            // in the last-level cache: 4,096 keys 1.97 -> 1.94 ms, 16,384 keys in bands of 2,601
-            // 5.39 -> 5.32 ms; beyond it even or slower (at two workgroups per CU: 8,192 keys even,
-            // 16,384 keys 40.8 -> 44.6 ms)
-            const bool e_store = (double) n_slots * (double) pl.slot_bytes <= (double) NXG_ATT_E_STORE_MIB * 1048576.0;
-            const dim3 grid((unsigned) n_slots), block(256);
-            float * const ws = (float *) workspace;
-            hipStream_t s = (hipStream_t) stream;
-            if (e_store && p.half >= 0) attention_stored_kernel<true, true><<<grid, block, 0, s>>>(p, ws);
-            else if (e_store)           attention_stored_kernel<true, false><<<grid, block, 0, s>>>(p, ws);
-            else if (p.half >= 0)       attention_stored_kernel<false, true><<<grid, block, 0, s>>>(p, ws);
-            else                        attention_stored_kernel<false, false><<<grid, block, 0, s>>>(p, ws);
-            return launch_check("attention_stored_kernel");
+        if (pl.lds_fits) {
+            attention_mfma_kernel<false><<<dim3((unsigned) pl.n_tiles), dim3(256), (size_t) pl.need * ATT_TILE_BYTES, s>>>(
+                p, pl.need, 0, nullptr);
+            return launch_check("attention_mfma_kernel");
         }
-        attention_long_kernel<<<dim3((unsigned) n_tiles), dim3(256), 0, (hipStream_t) stream>>>(p);
+        attention_long_kernel<<<dim3((unsigned) pl.n_tiles), dim3(256), 0, s>>>(p);
         return launch_check("attention_long_kernel");
     }
     if (max_keys > NXG_ATTN_MAX_KEYS) {

@@ -1,0 +1,92 @@
+"""GPU: attention on the matrix cores bit for bit against the oracle where its tiling can go
+wrong: key counts around the 16-key tile and the 8-key group, every head ratio that divides 16,
+bands narrower and wider than a tile, workgroups whose queries lie in several documents (also
+where those documents' scores do not fit together), scores split between LDS and a workspace of
+any size and alignment, and non-finite queries, keys and values."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    assert t.cuda.is_available(), "no GPU"
+    return t
+
+
+@pytest.fixture(scope="module")
+def dev(torch, nxg):
+    nxg.init()
+    return torch.device("cuda:0")
+
+
+def bits(a):
+    return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
+
+
+def check(nxg, orc, torch, lengths, half, H, G, workspaces=(None,), seed=0, spoil=None):
+    rng = np.random.default_rng(seed)
+    cu = nxg.cu_offsets_of(lengths)
+    T = int(cu[-1])
+    q = rng.standard_normal((T, H * 64)).astype(np.float32)
+    k, v = (rng.standard_normal((G, T, 64)).astype(np.float32) for _ in range(2))
+    scale = rng.uniform(0.05, 0.3, len(lengths)).astype(np.float32)
+    if spoil:
+        spoil(q, k, v)
+    ref = orc.attention(q, k, v, cu, scale, H, G, half)
+    dev = [torch.from_numpy(a).cuda() for a in (q, k, v)]
+    for ws in workspaces:
+        size = ws if ws is None or isinstance(ws, str) else ws.numel()
+        print(f"attention lengths={lengths} half={half} H={H} G={G} workspace={size}", flush=True)
+        y = nxg.attention(*dev, cu, scale, H, G, half, workspace=ws).cpu().numpy()
+        assert ((bits(y) == bits(ref)) | (np.isnan(y) & np.isnan(ref))).all()
+
+
+@pytest.mark.parametrize("H,G", [(4, 4), (4, 2), (4, 1), (8, 1), (16, 1)])
+@pytest.mark.parametrize("half", [-1, 0, 3, 8, 20])
+def test_tile_edges(nxg, orc, torch, dev, H, G, half):
+    check(nxg, orc, torch, [15, 16, 17, 1, 23, 24, 25, 33, 64, 7, 113], half, H, G, seed=H + half)
+
+
+@pytest.mark.parametrize("lengths,half,H,G", [
+    ([700, 900, 5, 820], -1, 4, 2),       # neighbours span more keys than the tiles hold
+    ([1290, 1283, 1296], -1, 2, 1),
+    ([1401, 1500], 640, 4, 4),
+    ([3100, 3, 2900], -1, 2, 1),
+    ([2700, 40], 1300, 16, 1),
+])
+def test_scores_in_lds_and_workspace(nxg, orc, torch, dev, lengths, half, H, G):
+    T, most = sum(lengths), max(lengths) if half < 0 else min(max(lengths), 2 * half + 1)
+    slot = 16 * most * 4
+    odd = torch.empty(5 * slot + 16, dtype=torch.uint8, device="cuda")[4:]    # 4-byte aligned only
+    one = torch.empty(slot, dtype=torch.uint8, device="cuda")
+    check(nxg, orc, torch, lengths, half, H, G, workspaces=(None, "auto", odd, one), seed=T)
+
+
+@pytest.mark.parametrize("half", [-1, 9])
+def test_non_finite_queries_keys_values(nxg, orc, torch, dev, half):
+    n = [40, 70, 21]
+
+    def nan_first_key(q, k, v):
+        k[0, 0, 3] = np.nan               # the first score of document 0: the maximum is NaN
+        k[1, 55, 60] = np.nan             # a later one: never the maximum
+    check(nxg, orc, torch, n, half, 8, 2, seed=1, spoil=nan_first_key)
+
+    def inf_key_and_query(q, k, v):
+        k[0, 12, 1] = np.inf
+        k[1, 90, 2] = -np.inf
+        q[44, 5] = np.inf
+        q[129, 7] = np.nan
+    check(nxg, orc, torch, n, half, 8, 2, seed=2, spoil=inf_key_and_query)
+
+    def values(q, k, v):
+        v[0, 0, 0], v[0, 39, 1], v[1, 40, 2], v[1, 130, 63] = np.inf, np.nan, -np.inf, np.nan
+    check(nxg, orc, torch, n, half, 8, 2, seed=3, spoil=values)
+
+    def tiny(q, k, v):
+        v *= np.float32(1e-38)            # sums among the subnormals
+    check(nxg, orc, torch, n, half, 8, 2, seed=4, spoil=tiny)
