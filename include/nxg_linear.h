@@ -230,6 +230,15 @@ NXG_API int32_t nxg_attention_noalloc(const float * q, const float * k, const fl
                                       int32_t n_seqs, const float * scale, int32_t T, int32_t n_head,
                                       int32_t n_kv_head, int32_t half, int32_t max_keys, float * out, void * stream);
 
+/* n 32-bit words of host memory to device memory in stream order, without waiting: no
+ * counterpart in the reference. For the small arrays that calls here take on the device
+ * (document offsets, scales): the words are read before the call returns and travel as
+ * launch arguments, 896 to a launch, where a copy from pageable memory would wait for the
+ * stream's earlier work.
+ *   src  host memory   dst  device memory, 4-byte aligned   n  at most NXG_UPLOAD_MAX_WORDS */
+#define NXG_UPLOAD_MAX_WORDS 3584
+NXG_API int32_t nxg_upload_words(const void * src, int32_t n, void * dst, void * stream);
+
 /* Sizing for nxg_attention_ws (no counterpart in the reference, whose op_attention keeps a
  * document's scores in host memory): the workspace it uses for these sizes: 0 when the launch does not need one,
  * else one slot per resident workgroup (a negative NXG_E* code for invalid sizes). */

@@ -83,6 +83,7 @@ def load_library(path: Optional[os.PathLike] = None) -> ctypes.CDLL:
         "nxg_attention": ([P, P, P, P, i32, P, i32, i32, i32, i32, i32, P, P], i32),
         "nxg_attention_ws": ([P, P, P, P, i32, P, i32, i32, i32, i32, i32, P, P, i64, P], i32),
         "nxg_attention_workspace_bytes": ([i32, i32, i32, i32], i64),
+        "nxg_upload_words": ([P, i32, P, P], i32),
         "nxg_attention_scales": ([P, i32, i32, i32, ctypes.c_float, ctypes.c_float, ctypes.c_float, P], i32),
         "nxg_qk_prep": ([P, P, P, P, P, i32, P, i32, i32, i32, i32, i32, P, P], i32),
         "nxg_head_major": ([P, i32, i32, i32, P, P], i32),
@@ -169,7 +170,7 @@ def _check(rc: int, what: str) -> None:
 
 
 def _np_ptr(a: Optional[np.ndarray]):
-    return None if a is None else a.ctypes.data
+    return None if a is None else a.__array_interface__["data"][0]
 
 
 # --- host side: load-time expansion ------------------------------------------------------------
@@ -243,10 +244,18 @@ def _torch():
     return torch
 
 
+def _raw_device() -> int:
+    return _torch()._C._cuda_getDevice()
+
+
+def _raw_stream(device: int) -> int:
+    return _torch()._C._cuda_getCurrentRawStream(device)
+
+
 def _stream_ptr(stream=None) -> Optional[int]:
-    torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream or None
+    if stream is not None:
+        return stream.cuda_stream or None
+    return _raw_stream(_raw_device()) or None     # torch.cuda.current_stream() without its Stream object
 
 
 def _order_on(stream, *tensors) -> None:
@@ -375,13 +384,28 @@ def _rows_arg(t, name, shape=None):
     return t
 
 
+UPLOAD_MAX_WORDS = 3584                 # NXG_UPLOAD_MAX_WORDS
+
+
+def _uploaded(a, device):
+    """A host array of 32-bit values as a device tensor, made on torch's current stream. Small ones go
+    by nxg_upload_words, which does not wait for the stream (torch.tensor's copy from pageable
+    memory does: 3 of them cost a 512-token attention mixer about 50 of its 160 us)."""
+    torch = _torch()
+    if a.ndim != 1 or a.size == 0 or a.size > UPLOAD_MAX_WORDS or device.index not in (None, _raw_device()):
+        return torch.tensor(a, device=device)
+    t = torch.empty(a.size, dtype=torch.int32 if a.dtype == np.int32 else torch.float32, device=device)
+    _check(load_library().nxg_upload_words(_np_ptr(a), a.size, t.data_ptr(), _stream_ptr()), "upload_words")
+    return t
+
+
 def _device_offsets(cu_offsets, device):
     """cu_offsets (host sequence or device int32 tensor) as a device int32 tensor."""
     torch = _torch()
     if isinstance(cu_offsets, torch.Tensor):
         t = cu_offsets.to(device=device, dtype=torch.int32).contiguous()
     else:
-        t = torch.tensor(np.ascontiguousarray(cu_offsets, dtype=np.int32), device=device)
+        t = _uploaded(np.ascontiguousarray(cu_offsets, dtype=np.int32), device)
     if t.dim() != 1 or t.numel() < 2:
         raise ValueError("cu_offsets: need n_seqs + 1 >= 2 offsets")
     return t
@@ -521,8 +545,10 @@ def attention(q, k, v, cu_offsets: Sequence[int], scale, n_head: int, n_kv_head:
     lens = np.diff(cu_host)
     max_keys = int(lens.max()) if half < 0 else int(min(lens.max(), 2 * half + 1))
     cu = _device_offsets(cu_host, q.device)
-    sc = scale if isinstance(scale, torch.Tensor) else torch.tensor(np.asarray(scale, np.float32), device=q.device)
-    sc = sc.to(device=q.device, dtype=torch.float32).contiguous()
+    if isinstance(scale, torch.Tensor):
+        sc = scale.to(device=q.device, dtype=torch.float32).contiguous()
+    else:
+        sc = _uploaded(np.ascontiguousarray(scale, np.float32), q.device)
     if out is None:
         out = torch.empty_like(q)
     if workspace is None:

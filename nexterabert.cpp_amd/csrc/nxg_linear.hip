@@ -1631,6 +1631,17 @@ __global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
     }
 }
 
+// Small host arrays (offsets, scales) on their way to the device: the words travel as the launch's
+// arguments, read when it is made, so the call neither copies nor waits for the stream. Latency
+// only: the blocking copy it takes the place of waited for everything before it on the stream.
+constexpr int UPLOAD_WORDS = 896;      // 3.5 KiB of a launch's 4 KiB of arguments
+struct upload_words {
+    uint32_t w[UPLOAD_WORDS];
+};
+__global__ __launch_bounds__(256) void upload_kernel(uint32_t * __restrict__ dst, int n, upload_words a) {
+    for (int i = (int) threadIdx.x; i < n; i += 256) dst[i] = a.w[i];
+}
+
 // tanh256 (src/nexterabert.cpp:103-117) lane by lane: big = (1 - t) / (1 + t) with t =
 // exp256(|x| * -2) and x's sign bit ORed in, small = the fused odd polynomial * x, small
 // where |x| < 0.1 (ordered: a NaN takes big).
@@ -3883,6 +3894,23 @@ int64_t nxg_attention_workspace_bytes(int32_t T, int32_t n_head, int32_t n_kv_he
     const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
     if (pl.kind != 1) return 0;
     return std::min(pl.n_tiles, attention_slots(pl.need)) * pl.slot_bytes;
+}
+
+int32_t nxg_upload_words(const void * src, int32_t n, void * dst, void * stream) {
+    if (n < 0 || n > NXG_UPLOAD_MAX_WORDS) return fail(NXG_EINVAL, "upload_words: n=%d (at most %d)", n, NXG_UPLOAD_MAX_WORDS);
+    if (n == 0) return NXG_OK;
+    if (!src || !dst || ((uintptr_t) dst & 3)) return fail(NXG_EINVAL, "upload_words: null or unaligned buffer");
+    int rc = check_device();
+    if (rc) return rc;
+    for (int o = 0; o < n; o += UPLOAD_WORDS) {
+        upload_words a;
+        const int m = std::min(UPLOAD_WORDS, n - o);
+        memcpy(a.w, (const uint32_t *) src + o, (size_t) m * sizeof(uint32_t));
+        upload_kernel<<<dim3(1), dim3(256), 0, (hipStream_t) stream>>>((uint32_t *) dst + o, m, a);
+        rc = launch_check("upload_kernel");
+        if (rc) return rc;
+    }
+    return NXG_OK;
 }
 
 int32_t nxg_attention_noalloc(const float * q, const float * k, const float * v, const int32_t * cu_offsets,
