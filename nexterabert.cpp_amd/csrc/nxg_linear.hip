@@ -367,8 +367,10 @@ __global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const float * __r
 // NaN anywhere in the group's normalized values sends the group through quantize_block,
 // whose fold gives the reference's MAXPS result; without NaN that fold is the plain max.
 // SPLIT (few rows): one workgroup per (row group, block), the dot still over the whole row
-// from registers, only one block quantized and stored -- NB times the workgroups for
-// launches too small to fill the device. Workgroup b runs on XCD b % 8, so the NB
+// from registers, only one block normalized, quantized and stored -- NB times the workgroups for
+// launches too small to fill the device. Latency: its own 8 pairs and their gains are loaded
+// with the row, and code for one block instead of a choice of NB, each fetched by a cold
+// launch, takes 125 or 1,024 rows of 1,024 from 5.5 to 4.5 us. Workgroup b runs on XCD b % 8, so the NB
 // workgroups of a row group are given the same b % 8 and share that XCD's L2 for the rows
 // they all read (the grid is padded to whole rounds of 8 row groups).
 template <int ACT_MAX, int NB, bool SPLIT>
@@ -376,21 +378,33 @@ __global__ __launch_bounds__(256) void rmsnorm_q8_kernel(const float * __restric
                                                          float eps, int T, int8_t * __restrict__ q,
                                                          float * __restrict__ sx) {
     constexpr int n_in = NB * BLK, M = n_in / 32, KS = 4 * NB;
-    __shared__ __attribute__((aligned(16))) int stage[KS * FRAG / 4];
+    __shared__ __attribute__((aligned(16))) int stage[(SPLIT ? 4 : KS) * FRAG / 4];
     const int xcd = (int) (blockIdx.x & 7u), slot = (int) (blockIdx.x >> 3);
     const int g = SPLIT ? (slot / NB) * 8 + xcd : (int) blockIdx.x;
     const int Bs = SPLIT ? slot % NB : 0;                      // SPLIT: the block of this workgroup
     if (SPLIT && g * 16 >= T) return;                          // padding of the grid to whole rounds
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int rl = wave * 4 + (lane >> 4), t = g * 16 + rl, c = lane & 15;
-    float2 v[M];
+    float2 v[M], own[8], own_gain[8];          // own: SPLIT, the block's pairs
     if (t < T) {
         const float * xr = x + (size_t) t * n_in + 2 * c;
+        if constexpr (SPLIT) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) own[i] = *reinterpret_cast<const float2 *>(xr + BLK * Bs + 32 * i);
+        }
 #pragma unroll
         for (int m = 0; m < M; ++m) v[m] = *reinterpret_cast<const float2 *>(xr + 32 * m);
     } else {
 #pragma unroll
         for (int m = 0; m < M; ++m) v[m] = float2{ 0.0f, 0.0f };
+        if constexpr (SPLIT) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) own[i] = float2{ 0.0f, 0.0f };
+        }
+    }
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) own_gain[i] = *reinterpret_cast<const float2 *>(gain + BLK * Bs + 32 * i + 2 * c);
     }
     float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
@@ -400,7 +414,44 @@ __global__ __launch_bounds__(256) void rmsnorm_q8_kernel(const float * __restric
     }
     const float dot = dot_tree16(a0, a1);
     const float inv = 1.0f / __builtin_sqrtf(dot / (float) n_in + eps);
+    const src_rms src{src_rows{x, n_in}, gain, inv};
+    unsigned short * st16 = reinterpret_cast<unsigned short *>(stage);
+    // a block's 8 pairs to int8, in fragment order from fragment f0 of the stage
+    auto block = [&](const float2 * vb, int B, int f0) {
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fmaxf(abs_bits(vb[i].x), abs_bits(vb[i].y)));
+#pragma unroll
+        for (int sft = 1; sft < 16; sft <<= 1) amax = fmaxf(amax, __shfl_xor(amax, sft));
+        const float scale = amax / (float) ACT_MAX;
+        const float qinv = amax > 0.0f ? (float) ACT_MAX / amax : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int kq = 32 * (i & 1) + 2 * c;
+            const int pair = (quant1<ACT_MAX>(vb[i].x, qinv) & 0xff) | ((quant1<ACT_MAX>(vb[i].y, qinv) & 0xff) << 8);
+            st16[((f0 + (i >> 1)) * FRAG + (rl + 16 * (kq >> 4)) * 16 + (kq & 15)) / 2] = (unsigned short) pair;
+        }
+        if (c == 0) sx[((size_t) (t >> 2) * NB + B) * 4 + (t & 3)] = t < T ? scale : 0.0f;
+    };
     bool nan = false;
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            own[i].x = (own[i].x * inv) * own_gain[i].x;
+            own[i].y = (own[i].y * inv) * own_gain[i].y;
+            nan |= __builtin_isnan(own[i].x) || __builtin_isnan(own[i].y);
+        }
+        if (__syncthreads_or(nan)) {
+            quantize_block<ACT_MAX>(src, T, n_in, KS, NB, q, sx, g, Bs, stage);
+            return;
+        }
+        block(own, Bs, 0);
+        __syncthreads();
+        // wave w stores fragment w of the block
+        const int4 w = reinterpret_cast<const int4 *>(stage)[wave * 64 + lane];
+        *reinterpret_cast<int4 *>(q + ((size_t) g * KS + 4 * Bs + wave) * FRAG + lane * 16) = w;
+        return;
+    }
 #pragma unroll
     for (int m = 0; m < M; ++m) {
         const float2 gv = *reinterpret_cast<const float2 *>(gain + 32 * m + 2 * c);
@@ -409,40 +460,15 @@ __global__ __launch_bounds__(256) void rmsnorm_q8_kernel(const float * __restric
         nan |= __builtin_isnan(v[m].x) || __builtin_isnan(v[m].y);
     }
     if (__syncthreads_or(nan)) {
-        const src_rms src{src_rows{x, n_in}, gain, inv};
         for (int B = 0; B < NB; ++B) {
-            if (SPLIT && B != Bs) continue;
             quantize_block<ACT_MAX>(src, T, n_in, KS, NB, q, sx, g, B, stage);
             __syncthreads();
         }
         return;
     }
-    unsigned short * st16 = reinterpret_cast<unsigned short *>(stage);
 #pragma unroll
-    for (int B = 0; B < NB; ++B) {
-        if (SPLIT && B != Bs) continue;
-        float amax = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fmaxf(abs_bits(v[8 * B + i].x), abs_bits(v[8 * B + i].y)));
-#pragma unroll
-        for (int sft = 1; sft < 16; sft <<= 1) amax = fmaxf(amax, __shfl_xor(amax, sft));
-        const float scale = amax / (float) ACT_MAX;
-        const float qinv = amax > 0.0f ? (float) ACT_MAX / amax : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int kq = 32 * (i & 1) + 2 * c;
-            const int pair = (quant1<ACT_MAX>(v[8 * B + i].x, qinv) & 0xff) | ((quant1<ACT_MAX>(v[8 * B + i].y, qinv) & 0xff) << 8);
-            st16[((4 * B + (i >> 1)) * FRAG + (rl + 16 * (kq >> 4)) * 16 + (kq & 15)) / 2] = (unsigned short) pair;
-        }
-        if (c == 0) sx[((size_t) (t >> 2) * NB + B) * 4 + (t & 3)] = t < T ? scale : 0.0f;
-    }
+    for (int B = 0; B < NB; ++B) block(v + 8 * B, B, 4 * B);
     __syncthreads();
-    if (SPLIT) {
-        const int f = 4 * Bs + wave;                       // wave w stores fragment w of the block
-        const int4 w = reinterpret_cast<const int4 *>(stage)[f * 64 + lane];
-        *reinterpret_cast<int4 *>(q + ((size_t) g * KS + f) * FRAG + lane * 16) = w;
-        return;
-    }
 #pragma unroll
     for (int f = wave; f < KS; f += 4) {
         const int4 w = reinterpret_cast<const int4 *>(stage)[f * 64 + lane];
