@@ -883,7 +883,8 @@ __device__ __forceinline__ bool finite4(const v4f & x) {
 //            a second c = 4..7; the 8 chains of a score end in one lane for the tree
 //   values   acc = fma(w_j, v_j[d], acc) over the keys in order: one MFMA takes four keys
 // A workgroup takes the ATT_P (query, head) pairs of ATT_P / rep consecutive query rows and one
-// KV head; a tile is 16 keys. Scores are computed transposed (keys are the MFMA's rows) with row
+// KV head (NP such groups, so that a key or value row is read once for all of them); a tile is
+// 16 keys. Scores are computed transposed (keys are the MFMA's rows) with row
 // 4g + r standing for key 4r + g, so that register r of lane (g = lane >> 4, pair = lane & 15)
 // is the score of key 4r + g: what every later phase wants without moving data between lanes:
 //   scores   the waves take the tiles in turn, 16 MFMAs each; a tile's 4 scores per lane are
@@ -911,7 +912,7 @@ constexpr int ATT_P = 16;              // (query, head) pairs per workgroup
 constexpr int ATT_TILE = 16;           // keys per tile
 constexpr int ATT_TILE_BYTES = ATT_P * ATT_TILE * 4;
 constexpr int ATT_VC = 4;              // tiles per step of the value loop
-constexpr int ATT_STATIC_LDS = 9216;   // LDS beside the tiles, at most
+constexpr int att_static_lds(int np) { return np == 1 ? 9216 : 10240; }   // LDS beside the tiles, at most
 constexpr int ATT_MAX_KEYS = 1 << 23;  // keys whose row offsets fit the buffer loads' 32 bits
 
 // the workspace is 4-byte aligned
@@ -966,7 +967,9 @@ __device__ __forceinline__ v4f bload16f(__amdgpu_buffer_rsrc_t r, uint32_t voff)
 }
 
 // WS: tiles past lds_tiles (a multiple of ATT_VC) live in the workgroup's slot of ws (ws_tiles
-// tiles each), and the grid is persistent.
+// tiles each), and the grid is persistent; with NP = 2 half the key and value traffic (one group ->
+// two: 16,384 keys 25.7 -> 23.2 ms, 32,768 keys 109 -> 94 ms), two workgroups of up to 256
+// registers per CU.
 //
 // What bounds it: an fp32 MFMA (32 cycles for 1,024 FMAs) keeps the vector unit's FMA rate, and
 // vector instructions do not hide under it (16 MFMAs with 2 or 8 vector instructions each on four
@@ -975,81 +978,117 @@ __device__ __forceinline__ v4f bload16f(__amdgpu_buffer_rsrc_t r, uint32_t voff)
 // and issue slots away: the same FMAs as vector
 // instructions, with their LDS reads and broadcasts, ran at about 30 TFLOP/s; this runs at 45-65. At most 128
 // registers, so that four workgroups share a CU: two took 181 us where four take 161 (8 x 1,024
-// tokens, band 256). Before -> now: 1,024 keys 178 -> 101 us, 8 x 1,024 tokens in bands of
-// 257 keys 279 -> 174 us, 32 documents of 16 to 2,048 tokens 7.45 -> 3.02 ms (with the launch).
+// tokens, band 256). Kernel times: 1,024 keys 75 us, 8 x 1,024 tokens
+// in bands of 257 keys 161 us, 32 documents of 16 to 2,048 tokens 2.81 ms (on the vector unit
+// about 150, 250 us and 7.4 ms).
 // Lane numbers are taken anew in each phase: kept across them, the addresses made from them cost
 // 50 registers.
-template <bool WS>
-__global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, int lds_tiles, int ws_tiles,
+template <bool WS, int NP>
+__global__ __launch_bounds__(256, NP == 1 ? 4 : 2) void attention_mfma_kernel(attn_params p, int lds_tiles, int ws_tiles,
                                                                            float * __restrict__ ws) {
     extern __shared__ __attribute__((aligned(16))) float att_lds[];
     __shared__ __attribute__((aligned(16))) float wbuf[4][512];   // each wave's own: keys or values in transit
-    __shared__ float mx_s[4][ATT_P], s0_s[ATT_P], inv_s[ATT_P], tail_s[ATT_P][8];
+    constexpr int PAIRS = ATT_P * NP;
+    __shared__ float mx_s[4][PAIRS], s0_s[PAIRS], inv_s[PAIRS], tail_s[PAIRS][8];
     const int lane = (int) threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
     const int g4 = lane >> 4, pi = lane & 15;
-    const int lg_rep = __builtin_ctz((unsigned) (p.H / p.G)), rep = 1 << lg_rep, nq = ATT_P >> lg_rep;
+    const int lg_rep = __builtin_ctz((unsigned) (p.H / p.G)), rep = 1 << lg_rep, nq = PAIRS >> lg_rep;
     const int n_tiles = p.G * ((p.T + nq - 1) / nq);
     const int cap = ATT_TILE * (lds_tiles + ws_tiles);
     // the wave that adds up: waves 0 of a CU's workgroups share a SIMD, so it goes by their slot
     // there (hwreg HW_ID's wave slot, 4 bits at 0)
     __shared__ int adder_s;
     if (threadIdx.x == 0) adder_s = __builtin_amdgcn_s_getreg(4 | (0 << 6) | (3 << 11)) & 3;
-    float * const slot = WS ? ws + (size_t) blockIdx.x * ws_tiles * (ATT_TILE_BYTES / 4) : nullptr;
-    // float x of tile i's scores, in LDS or in the slot
-    auto in_lds = [&](int i, int x) -> float * { return att_lds + i * 256 + x; };
-    auto in_slot = [&](int i, int x) -> float * { return slot + (size_t) (i - lds_tiles) * 256 + x; };
+    float * const slot = WS ? ws + (size_t) blockIdx.x * ws_tiles * (NP * ATT_TILE_BYTES / 4) : nullptr;
+    // float x of tile i's scores of pair group u, in LDS or in the slot
+    auto in_lds = [&](int i, int u, int x) -> float * { return att_lds + (i * NP + u) * 256 + x; };
+    auto in_slot = [&](int i, int u, int x) -> float * { return slot + ((size_t) (i - lds_tiles) * NP + u) * 256 + x; };
     // a lane's 4 scores of a tile known to be in LDS (lds_tag) or in the slot (slot_tag), or of any
     struct lds_tag {};
     struct slot_tag {};
-    auto t_load = [&](auto tag, int i, int x) -> v4f {
-        if constexpr (std::is_same_v<decltype(tag), lds_tag>) return *reinterpret_cast<const v4f *>(in_lds(i, x));
-        else return *reinterpret_cast<const v4f_u *>(in_slot(i, x));
+    auto t_load = [&](auto tag, int i, int u, int x) -> v4f {
+        if constexpr (std::is_same_v<decltype(tag), lds_tag>) return *reinterpret_cast<const v4f *>(in_lds(i, u, x));
+        else return *reinterpret_cast<const v4f_u *>(in_slot(i, u, x));
     };
-    auto t_store = [&](auto tag, int i, int x, v4f e) {
-        if constexpr (std::is_same_v<decltype(tag), lds_tag>) *reinterpret_cast<v4f *>(in_lds(i, x)) = e;
-        else *reinterpret_cast<v4f_u *>(in_slot(i, x)) = e;
+    auto t_store = [&](auto tag, int i, int u, int x, v4f e) {
+        if constexpr (std::is_same_v<decltype(tag), lds_tag>) *reinterpret_cast<v4f *>(in_lds(i, u, x)) = e;
+        else *reinterpret_cast<v4f_u *>(in_slot(i, u, x)) = e;
     };
-    auto s_load = [&](int i, int x) -> v4f {
-        return !WS || i < lds_tiles ? t_load(lds_tag{}, i, x) : t_load(slot_tag{}, i, x);
+    auto s_load = [&](int i, int u, int x) -> v4f {
+        return !WS || i < lds_tiles ? t_load(lds_tag{}, i, u, x) : t_load(slot_tag{}, i, u, x);
     };
-    auto s_store = [&](int i, int x, v4f e) {
-        if (!WS || i < lds_tiles) t_store(lds_tag{}, i, x, e);
-        else t_store(slot_tag{}, i, x, e);
+    auto s_store = [&](int i, int u, int x, v4f e) {
+        if (!WS || i < lds_tiles) t_store(lds_tag{}, i, u, x, e);
+        else t_store(slot_tag{}, i, u, x, e);
+    };
+    // the address of one score: key k of the workgroup's, pair group u, pair pi
+    auto one_score = [&](int k, int u, int pi) -> float * {
+        const int x = ((k & 3) * 16 + pi) * 4 + ((k & 15) >> 2);
+        return !WS || k / ATT_TILE < lds_tiles ? in_lds(k / ATT_TILE, u, x) : in_slot(k / ATT_TILE, u, x);
     };
 
     for (int bt = (int) blockIdx.x; bt < n_tiles; bt += (int) gridDim.x) {
         // the KV head changes fastest: with 8 of them each XCD's L2 serves one
         const int g = bt % p.G, t0 = (bt / p.G) * nq;
-        const int t = t0 + (pi >> lg_rep), h = (g << lg_rep) + (pi & (rep - 1));
-        doc_rows dr = doc_of_wave(p.cu, p.n_seqs, t0, min(t, p.T - 1), p.T, lane);
-        if (p.half >= 0) {
-            dr.lo = max(dr.lo, t - p.half);
-            dr.hi = (int) min((long long) dr.hi, (long long) t + p.half + 1);
-        }
-        const int lo = dr.lo, hi = dr.hi, n = hi - lo;
-        const bool valid = t < p.T && n > 0 && n <= p.max_keys;
-        const float scale = p.scale[dr.d];
-        if (t < p.T && !valid) {                           // no keys, or more than max_keys
-            const float nan = __uint_as_float(0x7fc00000u);
-            *reinterpret_cast<v4f_u *>(p.out + (size_t) t * p.H * 64 + (size_t) h * 64 + 16 * w + 4 * g4) =
-                v4f{ nan, nan, nan, nan };
-        }
-
-        bool todo = valid;
-        while (__any(todo)) {                              // the same in every wave
-            bool act = todo;
-            int kl = row_min(act ? lo : INT_MAX), kh = row_max(act ? hi : INT_MIN);
-            if (kh - kl > cap) {
-                const int d0 = row_min(todo ? dr.d : INT_MAX);
-                act = todo && dr.d == d0;
-                kl = row_min(act ? lo : INT_MAX);
-                kh = row_max(act ? hi : INT_MIN);
+        int lo[NP], hi[NP], doc[NP];
+        bool todo[NP];
+        float scale[NP];
+#pragma unroll
+        for (int u = 0; u < NP; ++u) {
+            const int pr = ATT_P * u + pi;
+            const int t = t0 + (pr >> lg_rep), h = (g << lg_rep) + (pr & (rep - 1));
+            doc_rows dr = doc_of_wave(p.cu, p.n_seqs, t0, min(t, p.T - 1), p.T, lane);
+            if (p.half >= 0) {
+                dr.lo = max(dr.lo, t - p.half);
+                dr.hi = (int) min((long long) dr.hi, (long long) t + p.half + 1);
             }
-            const int na = act ? n : 0, ng = na & ~7;
+            lo[u] = dr.lo;
+            hi[u] = dr.hi;
+            doc[u] = dr.d;
+            scale[u] = p.scale[dr.d];
+            todo[u] = t < p.T && dr.hi > dr.lo && dr.hi - dr.lo <= p.max_keys;
+            if (t < p.T && !todo[u]) {                     // no keys, or more than max_keys
+                const float nan = __uint_as_float(0x7fc00000u);
+                *reinterpret_cast<v4f_u *>(p.out + (size_t) t * p.H * 64 + (size_t) h * 64 + 16 * w + 4 * g4) =
+                    v4f{ nan, nan, nan, nan };
+            }
+        }
+        auto least = [&](auto f) {
+            int x = f(0);
+#pragma unroll
+            for (int u = 1; u < NP; ++u) x = min(x, f(u));
+            return row_min(x);
+        };
+        auto most = [&](auto f) {
+            int x = f(0);
+#pragma unroll
+            for (int u = 1; u < NP; ++u) x = max(x, f(u));
+            return row_max(x);
+        };
+
+        while (least([&](int u) { return todo[u] ? 0 : 1; }) == 0) {   // the same in every wave
+            bool act[NP];
+#pragma unroll
+            for (int u = 0; u < NP; ++u) act[u] = todo[u];
+            int kl = least([&](int u) { return act[u] ? lo[u] : INT_MAX; });
+            int kh = most([&](int u) { return act[u] ? hi[u] : INT_MIN; });
+            if (kh - kl > cap) {
+                const int d0 = least([&](int u) { return todo[u] ? doc[u] : INT_MAX; });
+#pragma unroll
+                for (int u = 0; u < NP; ++u) act[u] = todo[u] && doc[u] == d0;
+                kl = least([&](int u) { return act[u] ? lo[u] : INT_MAX; });
+                kh = most([&](int u) { return act[u] ? hi[u] : INT_MIN; });
+            }
+            int na[NP], ng[NP];
+#pragma unroll
+            for (int u = 0; u < NP; ++u) {
+                na[u] = act[u] ? hi[u] - lo[u] : 0;
+                ng[u] = na[u] & ~7;
+            }
             const int nt = (kh - kl + ATT_TILE - 1) / ATT_TILE;
             // clean tiles [c0, c1): past every pair's first key's tile, before any pair's tail keys or end
-            int c0 = (row_max(act ? lo : INT_MIN) - kl) / ATT_TILE + 1;
-            int c1 = (row_min(act ? lo + ng : INT_MAX) - kl) / ATT_TILE;
+            int c0 = (most([&](int u) { return act[u] ? lo[u] : INT_MIN; }) - kl) / ATT_TILE + 1;
+            int c1 = (least([&](int u) { return act[u] ? lo[u] + ng[u] : INT_MAX; }) - kl) / ATT_TILE;
             if (c1 <= c0) c0 = c1 = 0;
             const int n_edge = nt - (c1 - c0);             // the others, [0, c0) and [c1, nt), taken by number
             auto edge = [&](int d) { return d < c0 ? d : d - c0 + c1; };
@@ -1068,15 +1107,19 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                 float * const kw1 = wbuf[w] + ((8 + fr) ^ 1) * 32 + (fc ^ fr) * 4;
                 const float * const kr0 = wbuf[w] + (pi ^ (pi >> 3)) * 32 + ((2 * g4) ^ (pi & 7)) * 4;
                 const float * const kr1 = wbuf[w] + (pi ^ (pi >> 3)) * 32 + ((2 * g4 + 1) ^ (pi & 7)) * 4;
-                const float * const qrow = p.q + (size_t) min(t0 + (pi >> lg_rep), p.T - 1) * p.H * 64 +
-                                           (size_t) ((g << lg_rep) + (pi & (rep - 1))) * 64 + 8 * g4;
-                v4f qf[4];
-                qf[0] = *reinterpret_cast<const v4f_u *>(qrow);
-                qf[1] = *reinterpret_cast<const v4f_u *>(qrow + 4);
-                qf[2] = *reinterpret_cast<const v4f_u *>(qrow + 32);
-                qf[3] = *reinterpret_cast<const v4f_u *>(qrow + 36);
-                const int key0 = kl + g4 - lo;             // key 4r + g4 of tile i is the pair's key0 + 16 i + 4 r
-                float mx = -__builtin_inff();
+                v4f qf[NP][4];
+                float mx[NP];
+#pragma unroll
+                for (int u = 0; u < NP; ++u) {
+                    const int pr = ATT_P * u + pi;
+                    const float * const qrow = p.q + (size_t) min(t0 + (pr >> lg_rep), p.T - 1) * p.H * 64 +
+                                               (size_t) ((g << lg_rep) + (pr & (rep - 1))) * 64 + 8 * g4;
+                    qf[u][0] = *reinterpret_cast<const v4f_u *>(qrow);
+                    qf[u][1] = *reinterpret_cast<const v4f_u *>(qrow + 4);
+                    qf[u][2] = *reinterpret_cast<const v4f_u *>(qrow + 32);
+                    qf[u][3] = *reinterpret_cast<const v4f_u *>(qrow + 36);
+                    mx[u] = -__builtin_inff();
+                }
                 v4f raw[4];
                 auto fetch = [&](int i) {
                     uint32_t o = koff0 + (uint32_t) i * 4096u;
@@ -1101,7 +1144,7 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                     kf[3] = *reinterpret_cast<const v4f *>(kr1);
                     keep_order();
                 };
-                auto chains = [&](const v4f (&kf)[4], v4f (&a)[8]) {
+                auto chains = [&](const v4f (&kf)[4], const v4f (&qf)[4], v4f (&a)[8]) {
                     const v4f nz = { -0.0f, -0.0f, -0.0f, -0.0f };
 #pragma unroll
                     for (int l = 0; l < 8; ++l)
@@ -1110,7 +1153,7 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                     for (int l = 0; l < 8; ++l)
                         a[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[2 + (l >> 2)][l & 3], qf[2 + (l >> 2)][l & 3], a[l], 0, 0, 0);
                 };
-                auto tree = [&](const v4f (&a)[8]) {
+                auto tree = [&](const v4f (&a)[8], float scale) {
                     v4f s;
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
@@ -1118,44 +1161,55 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                     return s;
                 };
                 auto tile = [&](const v4f (&kf)[4], int i) {
-                    v4f a[8];
-                    chains(kf, a);
-                    const v4f s = tree(a);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[r]);
-                    s_store(i, lx, s);
+                    for (int u = 0; u < NP; ++u) {
+                        v4f a[8];
+                        chains(kf, qf[u], a);
+                        const v4f s = tree(a, scale[u]);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) mx[u] = fmaxf(mx[u], s[r]);
+                        s_store(i, u, lx, s);
+                    }
                 };
                 v4f ka[4];
-                if (c0 + w < c1) {
-                    fetch(c0 + w);
+                // a tile ahead throughout, the clean ones and then the edges (with a workspace, where
+                // the edges are few among many and the registers are short, not ahead of the edges)
+                auto ahead = [&](int i) { return WS || i < c1 ? i : edge(min(3 - w, n_edge - 1)); };
+                fetch(ahead(c0 + w));
 #pragma unroll 1
-                    for (int i = c0 + w; i < c1; i += 4) {
-                        turn(ka);
-                        fetch(i + 4);
-                        tile(ka, i);
-                    }
+                for (int i = c0 + w; i < c1; i += 4) {
+                    turn(ka);
+                    fetch(ahead(i + 4));
+                    tile(ka, i);
                 }
 #pragma unroll 1
                 for (int d = 3 - w; d < n_edge; d += 4) {
                     const int i = edge(d);
-                    fetch(i);
+                    if (WS) fetch(i);
                     turn(ka);
-                    v4f a[8];
-                    chains(ka, a);
-                    v4f s = tree(a);
+                    if (!WS) fetch(edge(min(d + 4, n_edge - 1)));
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int jr = key0 + ATT_TILE * i + 4 * r;
-                        const float st = (((a[0][r] + a[4][r]) + (a[2][r] + a[6][r])) + ((a[1][r] + a[5][r]) + (a[3][r] + a[7][r]))) * scale;
-                        if (jr >= ng) s[r] = st;
-                        if (jr >= 0 && jr < na) mx = fmaxf(mx, s[r]);
-                        if (act && jr == 0) s0_s[pi] = s[r];
+                    for (int u = 0; u < NP; ++u) {
+                        v4f a[8];
+                        chains(ka, qf[u], a);
+                        v4f s = tree(a, scale[u]);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int jr = kl + g4 - lo[u] + ATT_TILE * i + 4 * r;
+                            const float st = (((a[0][r] + a[4][r]) + (a[2][r] + a[6][r])) + ((a[1][r] + a[5][r]) + (a[3][r] + a[7][r]))) * scale[u];
+                            if (jr >= ng[u]) s[r] = st;
+                            if (jr >= 0 && jr < na[u]) mx[u] = fmaxf(mx[u], s[r]);
+                            if (act[u] && jr == 0) s0_s[ATT_P * u + pi] = s[r];
+                        }
+                        s_store(i, u, lx, s);
                     }
-                    s_store(i, lx, s);
                 }
-                mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
-                if (lane < ATT_P) mx_s[w][pi] = mx;
+#pragma unroll
+                for (int u = 0; u < NP; ++u) {
+                    mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], 16));
+                    mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], 32));
+                    if (lane < ATT_P) mx_s[w][ATT_P * u + pi] = mx[u];
+                }
             }
             __syncthreads();
 
@@ -1164,55 +1218,55 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
             // key j of a pair per lane of waves 2 and 3.
             {
                 const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane;
-                const float s0 = s0_s[pi];
-                const float mx = fmaxf(fmaxf(mx_s[0][pi], mx_s[1][pi]), fmaxf(mx_s[2][pi], mx_s[3][pi]));
-                const float m = __builtin_isnan(s0) ? s0 : mx;
-                const int key0 = kl + g4 - lo;
-                auto part = [&](auto tag, int a, int b) {  // tiles a, a + 4, ... below b
-                    if (a >= b) return;
-                    const int last = a + ((b - 1 - a) & ~3);
-                    v4f x[2], y[2];
-                    x[0] = t_load(tag, a, lx);
-                    x[1] = t_load(tag, min(a + 4, last), lx);
-                    for (int i = a; i < b; i += 8) {
-                        y[0] = t_load(tag, min(i + 8, last), lx);
-                        y[1] = t_load(tag, min(i + 12, last), lx);
-                        keep_order();
 #pragma unroll
-                        for (int u = 0; u < 2; ++u)
+                for (int u = 0; u < NP; ++u) {
+                    const int pr = ATT_P * u + pi;
+                    const float s0 = s0_s[pr];
+                    const float mx = fmaxf(fmaxf(mx_s[0][pr], mx_s[1][pr]), fmaxf(mx_s[2][pr], mx_s[3][pr]));
+                    const float m = __builtin_isnan(s0) ? s0 : mx;
+                    auto part = [&](auto tag, int a, int b) {  // tiles a, a + 4, ... below b
+                        if (a >= b) return;
+                        const int last = a + ((b - 1 - a) & ~3);
+                        v4f x[2], y[2];
 #pragma unroll
-                            for (int r = 0; r < 4; ++r) x[u][r] = exp_cephes(x[u][r] - m);
-                        t_store(tag, i, lx, x[0]);
-                        if (i + 4 < b) t_store(tag, i + 4, lx, x[1]);
-                        x[0] = y[0];
-                        x[1] = y[1];
+                        for (int k = 0; k < 2; ++k) x[k] = t_load(tag, min(a + 4 * k, last), u, lx);
+                        for (int i = a; i < b; i += 8) {
+#pragma unroll
+                            for (int k = 0; k < 2; ++k) y[k] = t_load(tag, min(i + 8 + 4 * k, last), u, lx);
+                            keep_order();
+#pragma unroll
+                            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) x[k][r] = exp_cephes(x[k][r] - m);
+#pragma unroll
+                            for (int k = 0; k < 2; ++k)
+                                if (k == 0 || i + 4 * k < b) t_store(tag, i + 4 * k, u, lx, x[k]);
+#pragma unroll
+                            for (int k = 0; k < 2; ++k) x[k] = y[k];
+                        }
+                    };
+                    if constexpr (WS) {
+                        const int cl = min(max(c0, lds_tiles), c1);
+                        part(lds_tag{}, c0 + w, cl);
+                        part(slot_tag{}, cl + ((c0 + w - cl) & 3), c1);
+                    } else {
+                        part(lds_tag{}, c0 + w, c1);
                     }
-                };
-                if constexpr (WS) {
-                    const int cl = min(max(c0, lds_tiles), c1);
-                    part(lds_tag{}, c0 + w, cl);
-                    part(slot_tag{}, cl + ((c0 + w - cl) & 3), c1);
-                } else {
-                    part(lds_tag{}, c0 + w, c1);
-                }
-                const int j = 4 * (w & 1) + g4;
-                if (w >= 2 && j < na - ng) {
-                    const int k = lo - kl + ng + j, x = ((k & 3) * 16 + pi) * 4 + ((k & 15) >> 2);
-                    const float s = !WS || k / ATT_TILE < lds_tiles ? *in_lds(k / ATT_TILE, x) : *in_slot(k / ATT_TILE, x);
-                    tail_s[pi][j] = expf_libm(s - m);
-                }
+                    const int j = 4 * (w & 1) + g4;
+                    if (w >= 2 && j < na[u] - ng[u]) tail_s[pr][j] = expf_libm(*one_score(lo[u] - kl + ng[u] + j, u, pi) - m);
 #pragma unroll 1
-                for (int d = 3 - w; d < n_edge; d += 4) {
-                    const int i = edge(d);
-                    v4f e = s_load(i, lx);
+                    for (int d = 3 - w; d < n_edge; d += 4) {
+                        const int i = edge(d);
+                        v4f e = s_load(i, u, lx);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int jr = key0 + ATT_TILE * i + 4 * r;
-                        const float x = exp_cephes(e[r] - m);
-                        if (jr < ng) e[r] = jr >= 0 ? x : -0.0f;
-                        else if (jr >= na) e[r] = -0.0f;
+                        for (int r = 0; r < 4; ++r) {
+                            const int jr = kl + g4 - lo[u] + ATT_TILE * i + 4 * r;
+                            const float x = exp_cephes(e[r] - m);
+                            if (jr < ng[u]) e[r] = jr >= 0 ? x : -0.0f;
+                            else if (jr >= na[u]) e[r] = -0.0f;
+                        }
+                        s_store(i, u, lx, e);
                     }
-                    s_store(i, lx, e);
                 }
             }
             // the first values, under way meanwhile
@@ -1220,7 +1274,7 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
             // a tile's 16 dimensions of this wave: key lane >> 2, 16-byte piece lane & 3
             const int vlane = lane_here();
             const uint32_t voff = (uint32_t) (vlane >> 2) * 256u + (uint32_t) w * 64u + (uint32_t) (vlane & 3) * 16u;
-            v4f va[ATT_VC], vb[ATT_VC], ea[ATT_VC], eb[ATT_VC];
+            v4f va[ATT_VC], vb[ATT_VC];
             auto v_fetch = [&](v4f (&v)[ATT_VC], int i0) {
 #pragma unroll
                 for (int u = 0; u < ATT_VC; ++u) {
@@ -1230,44 +1284,49 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                 }
                 keep_order();
             };
-            auto e_fetch = [&](auto tag, v4f (&e)[ATT_VC], int i0, int last, int lx) {
+            auto e_fetch = [&](auto tag, v4f (&e)[ATT_VC], int i0, int last, int u, int lx) {
 #pragma unroll
-                for (int u = 0; u < ATT_VC; ++u) e[u] = t_load(tag, min(i0 + u, last), lx);
+                for (int k = 0; k < ATT_VC; ++k) e[k] = t_load(tag, min(i0 + k, last), u, lx);
                 keep_order();
             };
             v_fetch(va, 0);
             __syncthreads();
 
             // 1 / sum
-            if (w == adder_s) {
-                const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane;
-                const int key0 = kl + g4 - lo;             // key 4r + g4 of tile i is the pair's key0 + 16 i + 4 r
+            if (const int u = (w - adder_s) & 3; u < NP) {
+                const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane, pr = ATT_P * u + pi;
+                int lo_u = lo[0], na_u = na[0], ng_u = ng[0];
+#pragma unroll
+                for (int k = 1; k < NP; ++k)
+                    if (u == k) { lo_u = lo[k]; na_u = na[k]; ng_u = ng[k]; }
                 float l0 = 0.0f, l1 = 0.0f;
                 auto add = [&](const v4f & e) { l0 = l0 + e.x; l1 = l1 + e.y; l0 = l0 + e.z; l1 = l1 + e.w; };
                 auto add_edges = [&](int a, int b) {       // without the tail keys
 #pragma unroll 1
                     for (int i = a; i < b; ++i) {
-                        v4f e = s_load(i, lx);
+                        v4f e = s_load(i, u, lx);
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
-                            if (key0 + ATT_TILE * i + 4 * r >= ng) e[r] = 0.0f;
+                            if (kl + g4 - lo_u + ATT_TILE * i + 4 * r >= ng_u) e[r] = 0.0f;
                         add(e);
                     }
                 };
                 auto part = [&](auto tag, int a, int b) {
+                    v4f ea[ATT_VC], eb[ATT_VC];
+                    auto batch = [&](v4f (&e)[ATT_VC], int i0) { e_fetch(tag, e, i0, b - 1, u, lx); };
                     int i = a;
                     if (i + 2 * ATT_VC <= b) {
-                        e_fetch(tag, ea, i, b - 1, lx);
+                        batch(ea, i);
                         for (; i + 2 * ATT_VC <= b; i += 2 * ATT_VC) {
-                            e_fetch(tag, eb, i + ATT_VC, b - 1, lx);
+                            batch(eb, i + ATT_VC);
 #pragma unroll
-                            for (int u = 0; u < ATT_VC; ++u) add(ea[u]);
-                            e_fetch(tag, ea, i + 2 * ATT_VC, b - 1, lx);
+                            for (int k = 0; k < ATT_VC; ++k) add(ea[k]);
+                            batch(ea, i + 2 * ATT_VC);
 #pragma unroll
-                            for (int u = 0; u < ATT_VC; ++u) add(eb[u]);
+                            for (int k = 0; k < ATT_VC; ++k) add(eb[k]);
                         }
                     }
-                    for (; i < b; ++i) add(t_load(tag, i, lx));
+                    for (; i < b; ++i) add(t_load(tag, i, u, lx));
                 };
                 add_edges(0, c0);
                 if constexpr (WS) {
@@ -1281,21 +1340,25 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                 float sum = l0 + l1;
                 sum = sum + __shfl_xor(sum, 32);
                 sum = sum + __shfl_xor(sum, 16);
-                for (int j = 0; j < na - ng; ++j) {
-                    const float e = tail_s[pi][j];
+                for (int j = 0; j < na_u - ng_u; ++j) {
+                    const float e = tail_s[pr][j];
                     sum = sum + e;
-                    const int k = lo - kl + ng + j, x = ((k & 3) * 16 + pi) * 4 + ((k & 15) >> 2);
-                    if (g4 == 0) *(!WS || k / ATT_TILE < lds_tiles ? in_lds(k / ATT_TILE, x) : in_slot(k / ATT_TILE, x)) = e;
+                    if (g4 == 0) *one_score(lo_u - kl + ng_u + j, u, pi) = e;
                 }
-                if (lane < ATT_P) inv_s[pi] = 1.0f / sum;
+                if (lane < ATT_P) inv_s[pr] = 1.0f / sum;
             }
             __syncthreads();
 
             // values
             {
                 const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane;
-                const float inv = inv_s[pi];
-                v4f acc = { 0.0f, 0.0f, 0.0f, 0.0f };
+                float inv[NP];
+                v4f acc[NP];
+#pragma unroll
+                for (int u = 0; u < NP; ++u) {
+                    inv[u] = inv_s[ATT_P * u + pi];
+                    acc[u] = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
+                }
                 // two tiles at a time through the wave's buffer: register r of a tile is key 4r + g4,
                 // dimension 16 w + pi
                 auto turn = [&](v4f (&v)[ATT_VC]) {
@@ -1313,12 +1376,17 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                     }
                 };
                 // tiles past the last: weight -0, value 0
-                auto tiles = [&](const v4f (&e)[ATT_VC], const v4f (&v)[ATT_VC], int i) {
+                auto tiles = [&](const v4f (&e)[NP][ATT_VC], const v4f (&v)[ATT_VC], int i) {
 #pragma unroll
-                    for (int u = 0; u < ATT_VC; ++u) {
-                        const v4f wt = e[u] * (i + u < nt ? inv : -0.0f);
+                    for (int k = 0; k < ATT_VC; ++k) {
+                        v4f wt[NP];
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[r], v[u][r], acc, 0, 0, 0);
+                        for (int u = 0; u < NP; ++u) wt[u] = e[u][k] * (i + k < nt ? inv[u] : -0.0f);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int u = 0; u < NP; ++u)
+                                acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[u][r], v[k][r], acc[u], 0, 0, 0);
                     }
                 };
                 turn(va);
@@ -1326,12 +1394,19 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                 int i = 0;
                 auto part = [&](auto tag, int b) {
                     if (i >= b) return;
-                    e_fetch(tag, ea, i, b - 1, lx);
+                    v4f ea[NP][ATT_VC], eb[NP][ATT_VC];
+#pragma unroll
+                    for (int u = 0; u < NP; ++u) e_fetch(tag, ea[u], i, b - 1, u, lx);
                     for (; i < b; i += ATT_VC) {
-                        e_fetch(tag, eb, i + ATT_VC, b - 1, lx);
+#pragma unroll
+                        for (int u = 0; u < NP; ++u) e_fetch(tag, eb[u], i + ATT_VC, b - 1, u, lx);
                         tiles(ea, va, i);
 #pragma unroll
-                        for (int u = 0; u < ATT_VC; ++u) { va[u] = vb[u]; ea[u] = eb[u]; }
+                        for (int k = 0; k < ATT_VC; ++k) {
+                            va[k] = vb[k];
+#pragma unroll
+                            for (int u = 0; u < NP; ++u) ea[u][k] = eb[u][k];
+                        }
                         turn(va);
                         v_fetch(vb, i + 2 * ATT_VC);
                     }
@@ -1342,38 +1417,42 @@ __global__ __launch_bounds__(256, 4) void attention_mfma_kernel(attn_params p, i
                 } else {
                     part(lds_tag{}, nt);
                 }
-                const uint32_t rows = (uint32_t) __ballot(act) & 0xffffu;
-                auto is_act = [&](int r) { return ((rows >> (4 * g4 + r)) & 1) != 0; };
-                bool bad = false;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) bad = bad || (is_act(r) && !__builtin_isfinite(acc[r]));
                 // an Inf or NaN value makes every pair's sum of its dimension Inf or NaN, whatever the
                 // weights, also for pairs that do not attend to it: key by key then
-                if (__any(bad)) {
-                    acc = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
-#pragma unroll 1
-                    for (int j = 0; j < ATT_TILE * nt; ++j) {
-                        const v4f e = s_load(j / ATT_TILE, lx) * inv;
-                        const int r = (j & 15) >> 2;
-                        const bool mine = (j & 3) == g4;
-                        const float wj = r < 2 ? (r == 0 ? e.x : e.y) : (r == 2 ? e.z : e.w);
-                        const float vj = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                            vr, (int) ((uint32_t) j * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0));
-                        const v4f one = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? wj : 0.0f, mine ? vj : -0.0f, acc, 0, 0, 0);
-                        const uint64_t in = __ballot(act && kl + j >= lo && kl + j < hi);
 #pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            if ((in >> (4 * g4 + k)) & 1) acc[k] = one[k];
+                for (int u = 0; u < NP; ++u) {
+                    const uint32_t rows = (uint32_t) __ballot(act[u]) & 0xffffu;
+                    auto is_act = [&](int r) { return ((rows >> (4 * g4 + r)) & 1) != 0; };
+                    bool bad = false;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) bad = bad || (is_act(r) && !__builtin_isfinite(acc[u][r]));
+                    if (__any(bad)) {
+                        acc[u] = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll 1
+                        for (int j = 0; j < ATT_TILE * nt; ++j) {
+                            const v4f e = s_load(j / ATT_TILE, u, lx) * inv[u];
+                            const int r = (j & 15) >> 2;
+                            const bool mine = (j & 3) == g4;
+                            const float wj = r < 2 ? (r == 0 ? e.x : e.y) : (r == 2 ? e.z : e.w);
+                            const float vj = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                vr, (int) ((uint32_t) j * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0));
+                            const v4f one = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? wj : 0.0f, mine ? vj : -0.0f, acc[u], 0, 0, 0);
+                            const uint64_t in = __ballot(act[u] && kl + j >= lo[u] && kl + j < hi[u]);
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+                                if ((in >> (4 * g4 + k)) & 1) acc[u][k] = one[k];
+                        }
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int pr = ATT_P * u + 4 * g4 + r;
+                        if (is_act(r))
+                            p.out[(size_t) (t0 + (pr >> lg_rep)) * p.H * 64 + (size_t) ((g << lg_rep) + (pr & (rep - 1))) * 64 + 16 * w + pi] = acc[u][r];
                     }
                 }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int pr = 4 * g4 + r;
-                    if (is_act(r))
-                        p.out[(size_t) (t0 + (pr >> lg_rep)) * p.H * 64 + (size_t) ((g << lg_rep) + (pr & (rep - 1))) * 64 + 16 * w + pi] = acc[r];
-                }
             }
-            todo = todo && !act;
+#pragma unroll
+            for (int u = 0; u < NP; ++u) todo[u] = todo[u] && !act[u];
             __syncthreads();                               // the scores and sums have been read
         }
     }
@@ -3635,16 +3714,18 @@ static size_t attention_lds_limit() {
         int v = 0;
         limit = 0;
         if (dev >= 0 &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > ATT_STATIC_LDS) {
-            const size_t want = (size_t) v - ATT_STATIC_LDS;
-            if (hipFuncSetAttribute((const void *) attention_mfma_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int) want) == hipSuccess &&
-                hipFuncSetAttribute((const void *) attention_mfma_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int) want) == hipSuccess) {
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > att_static_lds(2)) {
+            const size_t want = (size_t) v - att_static_lds(1);
+            auto allow = [](const void * f, size_t bytes) {
+                return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) bytes) == hipSuccess;
+            };
+            if (allow((const void *) attention_mfma_kernel<false, 1>, want) &&
+                allow((const void *) attention_mfma_kernel<true, 1>, want) &&
+                allow((const void *) attention_mfma_kernel<true, 2>, (size_t) v - att_static_lds(2))) {
                 limit = want;
             } else {
                 (void) hipGetLastError();
-                limit = 65536 - ATT_STATIC_LDS;
+                limit = 65536 - att_static_lds(1);
             }
         }
         limit_dev = dev;
@@ -3838,75 +3919,77 @@ static int scratch_of_device(void ** out) {
     return NXG_OK;
 }
 
-// Tiles of LDS a workgroup of attention_mfma_kernel<true> takes: those of four workgroups per CU;
-// of two past 4,096 keys, where the slots of four (4 MiB each at 65,536 keys) and the keys and
-// values they read at different times outgrow the caches (2,048 keys 265 us with four, 282 with
-// two; 4,096 keys 1.11 and 1.10 ms; 16,384 keys 26.7 and 26.0 ms; 65,536 keys 543 and 463 ms).
-static int attention_ws_lds_tiles(int need) {
-    const int per_cu = need <= 257 ? 4 : 2;
-    return ((int) ((attention_lds_limit() + ATT_STATIC_LDS) / per_cu - ATT_STATIC_LDS) / ATT_TILE_BYTES) & ~(ATT_VC - 1);
+// Key tiles of a workgroup of np groups of ATT_P pairs: its pairs attend to at most max_keys +
+// (its query rows - 1) keys of one document.
+static int attention_need(int32_t max_keys, int rep, int np) {
+    return (max_keys + np * ATT_P / rep - 1 + ATT_TILE - 1) / ATT_TILE;
 }
 
-// Workgroups of attention_mfma_kernel<true> resident at once on the current device (its compute
+// Of these, those in LDS beside a workspace slot: with two groups, two workgroups share a CU's LDS;
+// with one (a workspace too small for a slot of two) a workgroup takes all of it.
+static int attention_ws_lds_tiles(int np) {
+    const int lds = (int) attention_lds_limit() + att_static_lds(1);
+    return ((lds / np - att_static_lds(np)) / (np * ATT_TILE_BYTES)) & ~(ATT_VC - 1);
+}
+
+// Workgroups of attention_mfma_kernel<true, 2> resident at once on the current device (its compute
 // units x occupancy), each needing one workspace slot. Cached per thread for the device it was
 // computed on, like check_device's device check.
-static long long attention_slots(int need) {
+static long long attention_slots() {
     static thread_local long long slots = 0;
-    static thread_local int slots_dev = -1, slots_lds = -1;
-    const int lds_tiles = attention_ws_lds_tiles(need);
+    static thread_local int slots_dev = -1;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
         (void) hipGetLastError();
         dev = -1;
     }
-    if (dev < 0 || dev != slots_dev || lds_tiles != slots_lds) {
+    if (dev < 0 || dev != slots_dev) {
         int cus = 0, per_cu = 0;
         if (dev >= 0 &&
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attention_mfma_kernel<true>, 256,
-                                                         (size_t) lds_tiles * ATT_TILE_BYTES) == hipSuccess &&
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attention_mfma_kernel<true, 2>, 256,
+                                                         (size_t) attention_ws_lds_tiles(2) * 2 * ATT_TILE_BYTES) == hipSuccess &&
             cus > 0 && per_cu > 0) {
             slots = (long long) cus * per_cu;
         } else {
             (void) hipGetLastError();
-            slots = 256;
+            slots = 128;
         }
         slots_dev = dev;
-        slots_lds = lds_tiles;
     }
     return slots;
 }
 
 // The launch nxg_attention_ws makes for (T, heads, max_keys): 0 the scores in LDS, 1 in LDS and a
 // workspace slot given one (else in LDS where they fit, else the recomputing long kernel), 2 row
-// kernel; the workgroups' tiles, the key tiles of one, the bytes of one slot, and whether all key
-// tiles fit in LDS.
+// kernel; the groups of ATT_P pairs, the key tiles of one, the workspace bytes a group may take, and
+// whether all key tiles fit in LDS.
 struct attn_plan {
     int kind;
-    long long n_tiles;
+    long long n_groups;
     int need;
-    long long slot_bytes;
+    long long group_bytes;
     bool lds_fits;
 };
 
-// A workgroup's pairs attend to at most max_keys + (its query rows - 1) keys of one document.
-// Where their LDS leaves room for one workgroup per CU, or for two while the launch has more
-// than two rounds of them, the workspace keeps what is past a quarter of a CU's LDS, so that four
-// run: 8 x 1,024 keys 564 -> 516 us, 2,048 keys 357 -> 265 us. Otherwise the scores stay in LDS
-// (512 keys 24.8 us, 25.4 with a workspace).
+// Where a group's tiles leave room for one workgroup per CU, or for two while the launch has more
+// than two rounds of them, two groups a workgroup with a workspace are faster: 8 x 1,024 keys
+// 560 -> 487 us, 2,048 keys 365 -> 264 us, 32 documents of 16 to 2,048 tokens 4.04 -> 2.81 ms (one
+// group a workgroup with a workspace: 512, 277 us, 2.96 ms). Otherwise the scores stay in LDS (512
+// keys 24.1 us, 27.0 with a workspace).
 static attn_plan plan_attention(int32_t T, int32_t n_head, int32_t n_kv_head, int32_t max_keys) {
     const int rep = n_head / n_kv_head;
     if (ATT_P % rep != 0) return {2, 0, 0, 0, false};
     const int nq = ATT_P / rep;
-    const long long n_tiles = (long long) n_kv_head * ((T + nq - 1) / nq);
-    const long long slot_bytes = (long long) ATT_P * max_keys * (long long) sizeof(float);
-    if (max_keys > ATT_MAX_KEYS) return {1, n_tiles, 0, slot_bytes, false};
-    const int need = (max_keys + nq - 1 + ATT_TILE - 1) / ATT_TILE;
+    const long long n_groups = (long long) n_kv_head * ((T + nq - 1) / nq);
+    const long long group_bytes = (long long) ATT_P * max_keys * (long long) sizeof(float);
+    if (max_keys > ATT_MAX_KEYS) return {1, n_groups, 0, group_bytes, false};
+    const int need = attention_need(max_keys, rep, 1);
     const size_t lds = (size_t) need * ATT_TILE_BYTES, lds_max = attention_lds_limit();
-    if (lds > lds_max) return {1, n_tiles, need, slot_bytes, false};
-    const size_t per_cu = (lds_max + ATT_STATIC_LDS) / (lds + ATT_STATIC_LDS);
-    const bool lds_first = per_cu >= 3 || (per_cu == 2 && n_tiles <= 4LL * device_cus());
-    return {lds_first ? 0 : 1, n_tiles, need, slot_bytes, true};
+    if (lds > lds_max) return {1, n_groups, need, group_bytes, false};
+    const size_t per_cu = (lds_max + att_static_lds(1)) / (lds + att_static_lds(1));
+    const bool lds_first = per_cu >= 3 || (per_cu == 2 && n_groups <= 4LL * device_cus());
+    return {lds_first ? 0 : 1, n_groups, need, group_bytes, true};
 }
 
 int64_t nxg_attention_workspace_bytes(int32_t T, int32_t n_head, int32_t n_kv_head, int32_t max_keys) {
@@ -3919,7 +4002,7 @@ int64_t nxg_attention_workspace_bytes(int32_t T, int32_t n_head, int32_t n_kv_he
     if (rc) return rc;
     const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
     if (pl.kind != 1) return 0;
-    return std::min(pl.n_tiles, attention_slots(pl.need)) * pl.slot_bytes;
+    return std::min(pl.n_groups, 2 * attention_slots()) * pl.group_bytes;
 }
 
 int32_t nxg_upload_words(const void * src, int32_t n, void * dst, void * stream) {
@@ -3950,11 +4033,11 @@ int32_t nxg_attention_noalloc(const float * q, const float * k, const float * v,
     int rc = check_device();
     if (rc) return rc;
     const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
-    const bool use_scratch = pl.kind == 1 && pl.slot_bytes <= (long long) NXG_NOALLOC_SCRATCH_BYTES;
+    const bool use_scratch = pl.kind == 1 && pl.group_bytes <= (long long) NXG_NOALLOC_SCRATCH_BYTES;
     if (pl.kind == 1 && !use_scratch && !pl.lds_fits) {
         return fail(NXG_EINVAL,
                     "attention_noalloc: max_keys=%d needs %lld bytes per workgroup's scores; the static scratch "
-                    "holds %lld (at most %lld keys)", max_keys, pl.slot_bytes, (long long) NXG_NOALLOC_SCRATCH_BYTES,
+                    "holds %lld (at most %lld keys)", max_keys, pl.group_bytes, (long long) NXG_NOALLOC_SCRATCH_BYTES,
                     (long long) NXG_NOALLOC_SCRATCH_BYTES / (ATT_P * (long long) sizeof(float)));
     }
     void * ws = nullptr;                       // none: the scores in LDS
@@ -3996,22 +4079,28 @@ int32_t nxg_attention_ws(const float * q, const float * k, const float * v, cons
     if (pl.kind != 2) {
         hipStream_t s = (hipStream_t) stream;
         if (pl.kind == 1 && pl.need > 0) {
-            // as many slots as the workspace holds, up to the resident workgroups
-            const int lds_tiles = attention_ws_lds_tiles(pl.need), ws_tiles = std::max(pl.need - lds_tiles, 1);
-            const long long n_slots = std::min({pl.n_tiles, attention_slots(pl.need),
-                                                (long long) (workspace_bytes / ((long long) ws_tiles * ATT_TILE_BYTES))});
-            if (n_slots >= 1) {
-                attention_mfma_kernel<true><<<dim3((unsigned) n_slots), dim3(256), (size_t) lds_tiles * ATT_TILE_BYTES, s>>>(
-                    p, lds_tiles, ws_tiles, (float *) workspace);
+            // as many slots as the workspace holds, up to the resident workgroups: of two groups,
+            // or of one where it holds none of two
+            for (int np = 2; np >= 1; --np) {
+                const int lds_tiles = attention_ws_lds_tiles(np);
+                const int ws_tiles = std::max(attention_need(max_keys, rep, np) - lds_tiles, 1);
+                const long long n_wg_all = (long long) n_kv_head * ((T + np * ATT_P / rep - 1) / (np * ATT_P / rep));
+                const long long n_slots = std::min({n_wg_all, attention_slots(),
+                                                    (long long) (workspace_bytes / ((long long) ws_tiles * np * ATT_TILE_BYTES))});
+                if (n_slots < 1) continue;
+                const dim3 grid((unsigned) n_slots), block(256);
+                const size_t lds = (size_t) lds_tiles * np * ATT_TILE_BYTES;
+                if (np == 2) attention_mfma_kernel<true, 2><<<grid, block, lds, s>>>(p, lds_tiles, ws_tiles, (float *) workspace);
+                else         attention_mfma_kernel<true, 1><<<grid, block, lds, s>>>(p, lds_tiles, ws_tiles, (float *) workspace);
                 return launch_check("attention_mfma_kernel");
             }
         }
         if (pl.lds_fits) {
-            attention_mfma_kernel<false><<<dim3((unsigned) pl.n_tiles), dim3(256), (size_t) pl.need * ATT_TILE_BYTES, s>>>(
+            attention_mfma_kernel<false, 1><<<dim3((unsigned) pl.n_groups), dim3(256), (size_t) pl.need * ATT_TILE_BYTES, s>>>(
                 p, pl.need, 0, nullptr);
             return launch_check("attention_mfma_kernel");
         }
-        attention_long_kernel<<<dim3((unsigned) pl.n_tiles), dim3(256), 0, s>>>(p);
+        attention_long_kernel<<<dim3((unsigned) pl.n_groups), dim3(256), 0, s>>>(p);
         return launch_check("attention_long_kernel");
     }
     if (max_keys > NXG_ATTN_MAX_KEYS) {
