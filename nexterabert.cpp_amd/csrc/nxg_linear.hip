@@ -969,7 +969,8 @@ __device__ __forceinline__ v4f bload16f(__amdgpu_buffer_rsrc_t r, uint32_t voff)
 // WS: tiles past lds_tiles (a multiple of ATT_VC) live in the workgroup's slot of ws (ws_tiles
 // tiles each), and the grid is persistent; with NP = 2 half the key and value traffic (one group ->
 // two: 16,384 keys 25.7 -> 23.2 ms, 32,768 keys 109 -> 94 ms), two workgroups of up to 256
-// registers per CU.
+// registers per CU. 65,536 keys 538 -> 375 ms in all: K, V and the scores' five passes through the
+// slot move about 13 TB/s through the L2s and 2.3 TB/s of HBM, and the phases wait on them.
 //
 // What bounds it: an fp32 MFMA (32 cycles for 1,024 FMAs) keeps the vector unit's FMA rate, and
 // vector instructions do not hide under it (16 MFMAs with 2 or 8 vector instructions each on four
@@ -979,12 +980,12 @@ __device__ __forceinline__ v4f bload16f(__amdgpu_buffer_rsrc_t r, uint32_t voff)
 // instructions, with their LDS reads and broadcasts, ran at about 30 TFLOP/s; this runs at 45-65. At most 128
 // registers, so that four workgroups share a CU: two took 181 us where four take 161 (8 x 1,024
 // tokens, band 256). Kernel times: 1,024 keys 75 us, 8 x 1,024 tokens
-// in bands of 257 keys 161 us, 32 documents of 16 to 2,048 tokens 2.81 ms (on the vector unit
+// in bands of 257 keys 161 us, 32 documents of 16 to 2,048 tokens 2.80 ms (on the vector unit
 // about 150, 250 us and 7.4 ms).
 // Lane numbers are taken anew in each phase: kept across them, the addresses made from them cost
 // 50 registers.
 template <bool WS, int NP>
-__global__ __launch_bounds__(256, NP == 1 ? 4 : 2) void attention_mfma_kernel(attn_params p, int lds_tiles, int ws_tiles,
+__global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_params p, int lds_tiles, int ws_tiles,
                                                                            float * __restrict__ ws) {
     extern __shared__ __attribute__((aligned(16))) float att_lds[];
     __shared__ __attribute__((aligned(16))) float wbuf[4][512];   // each wave's own: keys or values in transit
@@ -1048,7 +1049,8 @@ __global__ __launch_bounds__(256, NP == 1 ? 4 : 2) void attention_mfma_kernel(at
             scale[u] = p.scale[dr.d];
             todo[u] = t < p.T && dr.hi > dr.lo && dr.hi - dr.lo <= p.max_keys;
             if (t < p.T && !todo[u]) {                     // no keys, or more than max_keys
-                const float nan = __uint_as_float(0x7fc00000u);
+                float nan = __uint_as_float(0x7fc00000u);
+                asm volatile("" : "+v"(nan));              // made here, not kept through the loop
                 *reinterpret_cast<v4f_u *>(p.out + (size_t) t * p.H * 64 + (size_t) h * 64 + 16 * w + 4 * g4) =
                     v4f{ nan, nan, nan, nan };
             }
@@ -1172,8 +1174,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 4 : 2) void attention_mfma_kernel(at
                     }
                 };
                 v4f ka[4];
-                // a tile ahead throughout, the clean ones and then the edges (with a workspace, where
-                // the edges are few among many and the registers are short, not ahead of the edges)
+                // a tile ahead, the clean ones and the first edge (not where the edges are few among many)
                 auto ahead = [&](int i) { return WS || i < c1 ? i : edge(min(3 - w, n_edge - 1)); };
                 fetch(ahead(c0 + w));
 #pragma unroll 1
@@ -1185,9 +1186,8 @@ __global__ __launch_bounds__(256, NP == 1 ? 4 : 2) void attention_mfma_kernel(at
 #pragma unroll 1
                 for (int d = 3 - w; d < n_edge; d += 4) {
                     const int i = edge(d);
-                    if (WS) fetch(i);
+                    if (WS || d >= 4) fetch(i);
                     turn(ka);
-                    if (!WS) fetch(edge(min(d + 4, n_edge - 1)));
 #pragma unroll
                     for (int u = 0; u < NP; ++u) {
                         v4f a[8];
@@ -1247,8 +1247,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 4 : 2) void attention_mfma_kernel(at
                     };
                     if constexpr (WS) {
                         const int cl = min(max(c0, lds_tiles), c1);
-                        part(lds_tag{}, c0 + w, cl);
-                        part(slot_tag{}, cl + ((c0 + w - cl) & 3), c1);
+                        part(lds_tag{}, c0 + w, cl);   // the slot's below
                     } else {
                         part(lds_tag{}, c0 + w, c1);
                     }
@@ -1269,6 +1268,107 @@ __global__ __launch_bounds__(256, NP == 1 ? 4 : 2) void attention_mfma_kernel(at
                     }
                 }
             }
+            auto e_fetch = [&](auto tag, v4f (&e)[ATT_VC], int i0, int last, int u, int lx) {
+#pragma unroll
+                for (int k = 0; k < ATT_VC; ++k) e[k] = t_load(tag, min(i0 + k, last), u, lx);
+                keep_order();
+            };
+            // the ordered sums of group u = (w - adder) & 3, if there is one, are this wave's: l0, l1
+            const int au = (w - __builtin_amdgcn_readfirstlane(adder_s)) & 3;
+            float l0 = 0.0f, l1 = 0.0f;
+            auto pick = [&](const int (&x)[NP]) {
+                int y = x[0];
+#pragma unroll
+                for (int u = 1; u < NP; ++u) y = au == u ? x[u] : y;
+                return y;
+            };
+            auto add = [&](const v4f & e) { l0 = l0 + e.x; l1 = l1 + e.y; l0 = l0 + e.z; l1 = l1 + e.w; };
+            auto add_edges = [&](int a, int b, int lane) {     // without the tail keys
+                const int jr0 = kl + (lane >> 4) - pick(lo), ng_u = pick(ng);
+#pragma unroll 1
+                for (int i = a; i < b; ++i) {
+                    v4f e = s_load(i, au, 4 * lane);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (jr0 + ATT_TILE * i + 4 * r >= ng_u) e[r] = 0.0f;
+                    add(e);
+                }
+            };
+            auto add_part = [&](auto tag, int a, int b, int lx) {
+                v4f ea[ATT_VC], eb[ATT_VC];
+                auto batch = [&](v4f (&e)[ATT_VC], int i0) { e_fetch(tag, e, i0, b - 1, au, lx); };
+                int i = a;
+                if (i + 2 * ATT_VC <= b) {
+                    batch(ea, i);
+                    for (; i + 2 * ATT_VC <= b; i += 2 * ATT_VC) {
+                        batch(eb, i + ATT_VC);
+#pragma unroll
+                        for (int k = 0; k < ATT_VC; ++k) add(ea[k]);
+                        batch(ea, i + 2 * ATT_VC);
+#pragma unroll
+                        for (int k = 0; k < ATT_VC; ++k) add(eb[k]);
+                    }
+                }
+                for (; i < b; ++i) add(t_load(tag, i, au, lx));
+            };
+            int summed = 0;                                // tiles added
+            if constexpr (WS) {
+                // the slot's tiles 8 at a time, the sums a step behind: their reads wait for memory
+                // while the wave computes, not by themselves, and each score is read from the
+                // slot while it is near (32,768 keys 94.2 -> 88.6 ms, 2,048 keys 264 -> 247 us)
+                constexpr int STEP = 8, OWN = STEP / 4;
+                const int cl = min(max(c0, lds_tiles), c1);
+                if (cl < c1) {
+                    const int lane = lane_here(), pi = lane & 15, lx = 4 * lane;
+                    __syncthreads();                       // the exponentials of the tiles in LDS and the edges
+                    float m[NP];
+                    v4f x[NP][OWN], y[NP][OWN], e[STEP];
+#pragma unroll
+                    for (int u = 0; u < NP; ++u) {
+                        const int pr = ATT_P * u + pi;
+                        const float s0 = s0_s[pr];
+                        m[u] = fmaxf(fmaxf(mx_s[0][pr], mx_s[1][pr]), fmaxf(mx_s[2][pr], mx_s[3][pr]));
+                        if (__builtin_isnan(s0)) m[u] = s0;
+#pragma unroll
+                        for (int k = 0; k < OWN; ++k) x[u][k] = t_load(slot_tag{}, min(cl + w + 4 * k, c1 - 1), u, lx);
+                    }
+                    if (au < NP) {
+                        add_edges(0, c0, lane);
+                        add_part(lds_tag{}, c0, cl, lx);
+                    }
+                    for (int b = cl; b < c1; b += STEP) {
+#pragma unroll
+                        for (int u = 0; u < NP; ++u)
+#pragma unroll
+                            for (int k = 0; k < OWN; ++k)
+                                y[u][k] = t_load(slot_tag{}, min(b + STEP + w + 4 * k, c1 - 1), u, lx);
+                        const bool adds = au < NP && b > cl;
+                        if (adds) {
+#pragma unroll
+                            for (int k = 0; k < STEP; ++k) e[k] = t_load(slot_tag{}, b - STEP + k, au, lx);
+                        }
+                        keep_order();
+#pragma unroll
+                        for (int u = 0; u < NP; ++u)
+#pragma unroll
+                            for (int k = 0; k < OWN; ++k) {
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) x[u][k][r] = exp_cephes(x[u][k][r] - m[u]);
+                                if (b + w + 4 * k < c1) t_store(slot_tag{}, b + w + 4 * k, u, lx, x[u][k]);
+                            }
+                        if (adds) {
+#pragma unroll
+                            for (int k = 0; k < STEP; ++k) add(e[k]);
+                        }
+#pragma unroll
+                        for (int u = 0; u < NP; ++u)
+#pragma unroll
+                            for (int k = 0; k < OWN; ++k) x[u][k] = y[u][k];
+                        __syncthreads();                   // this step's exponentials
+                        summed = b;
+                    }
+                }
+            }
             // the first values, under way meanwhile
             const __amdgpu_buffer_rsrc_t vr = buffer_rsrc(p.v + ((size_t) g * p.T + kl) * 64, kv_bytes);
             // a tile's 16 dimensions of this wave: key lane >> 2, 16-byte piece lane & 3
@@ -1284,66 +1384,28 @@ __global__ __launch_bounds__(256, NP == 1 ? 4 : 2) void attention_mfma_kernel(at
                 }
                 keep_order();
             };
-            auto e_fetch = [&](auto tag, v4f (&e)[ATT_VC], int i0, int last, int u, int lx) {
-#pragma unroll
-                for (int k = 0; k < ATT_VC; ++k) e[k] = t_load(tag, min(i0 + k, last), u, lx);
-                keep_order();
-            };
             v_fetch(va, 0);
             __syncthreads();
 
             // 1 / sum
-            if (const int u = (w - adder_s) & 3; u < NP) {
-                const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane, pr = ATT_P * u + pi;
-                int lo_u = lo[0], na_u = na[0], ng_u = ng[0];
-#pragma unroll
-                for (int k = 1; k < NP; ++k)
-                    if (u == k) { lo_u = lo[k]; na_u = na[k]; ng_u = ng[k]; }
-                float l0 = 0.0f, l1 = 0.0f;
-                auto add = [&](const v4f & e) { l0 = l0 + e.x; l1 = l1 + e.y; l0 = l0 + e.z; l1 = l1 + e.w; };
-                auto add_edges = [&](int a, int b) {       // without the tail keys
-#pragma unroll 1
-                    for (int i = a; i < b; ++i) {
-                        v4f e = s_load(i, u, lx);
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            if (kl + g4 - lo_u + ATT_TILE * i + 4 * r >= ng_u) e[r] = 0.0f;
-                        add(e);
-                    }
-                };
-                auto part = [&](auto tag, int a, int b) {
-                    v4f ea[ATT_VC], eb[ATT_VC];
-                    auto batch = [&](v4f (&e)[ATT_VC], int i0) { e_fetch(tag, e, i0, b - 1, u, lx); };
-                    int i = a;
-                    if (i + 2 * ATT_VC <= b) {
-                        batch(ea, i);
-                        for (; i + 2 * ATT_VC <= b; i += 2 * ATT_VC) {
-                            batch(eb, i + ATT_VC);
-#pragma unroll
-                            for (int k = 0; k < ATT_VC; ++k) add(ea[k]);
-                            batch(ea, i + 2 * ATT_VC);
-#pragma unroll
-                            for (int k = 0; k < ATT_VC; ++k) add(eb[k]);
-                        }
-                    }
-                    for (; i < b; ++i) add(t_load(tag, i, u, lx));
-                };
-                add_edges(0, c0);
-                if constexpr (WS) {
-                    const int cl = min(max(c0, lds_tiles), c1);
-                    part(lds_tag{}, c0, cl);
-                    part(slot_tag{}, cl, c1);
-                } else {
-                    part(lds_tag{}, c0, c1);
+            if (au < NP) {
+                const int lane = lane_here(), pi = lane & 15, g4 = lane >> 4, lx = 4 * lane, pr = ATT_P * au + pi;
+                if (summed == 0) {
+                    add_edges(0, c0, lane);
+                    add_part(lds_tag{}, c0, WS ? min(max(c0, lds_tiles), c1) : c1, lx);
                 }
-                add_edges(c1, nt);
+                if constexpr (WS) {
+                    if (summed > 0) add_part(slot_tag{}, summed, c1, lx);
+                }
+                add_edges(c1, nt, lane);
+                const int lo_u = pick(lo), na_u = pick(na), ng_u = pick(ng);
                 float sum = l0 + l1;
                 sum = sum + __shfl_xor(sum, 32);
                 sum = sum + __shfl_xor(sum, 16);
                 for (int j = 0; j < na_u - ng_u; ++j) {
                     const float e = tail_s[pr][j];
                     sum = sum + e;
-                    if (g4 == 0) *one_score(lo_u - kl + ng_u + j, u, pi) = e;
+                    if (g4 == 0) *one_score(lo_u - kl + ng_u + j, au, pi) = e;
                 }
                 if (lane < ATT_P) inv_s[pr] = 1.0f / sum;
             }
@@ -3974,7 +4036,7 @@ struct attn_plan {
 
 // Where a group's tiles leave room for one workgroup per CU, or for two while the launch has more
 // than two rounds of them, two groups a workgroup with a workspace are faster: 8 x 1,024 keys
-// 560 -> 487 us, 2,048 keys 365 -> 264 us, 32 documents of 16 to 2,048 tokens 4.04 -> 2.81 ms (one
+// 548 -> 469 us, 2,048 keys 362 -> 247 us, 32 documents of 16 to 2,048 tokens 4.03 -> 2.80 ms (one
 // group a workgroup with a workspace: 512, 277 us, 2.96 ms). Otherwise the scores stay in LDS (512
 // keys 24.1 us, 27.0 with a workspace).
 static attn_plan plan_attention(int32_t T, int32_t n_head, int32_t n_kv_head, int32_t max_keys) {
