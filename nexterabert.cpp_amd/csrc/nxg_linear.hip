@@ -490,8 +490,6 @@ __global__ __launch_bounds__(256) void rmsnorm_q8_kernel(const float * __restric
 // Mixer producers quantizing for an int8 consumer (row_op(..., int8_only(...)))
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ float minps1(float a, float b) { return a < b ? a : b; }
-
 // exp(x) as the reference's exp256 computes it (src/nexterabert.cpp:81-100), lane by
 // lane: clamp to [-87.3, 88.3762626647949] with MINPS/MAXPS semantics (a NaN becomes the
 // upper bound); n = x * log2(e) rounded to the nearest integer (ties to even); the
@@ -618,6 +616,29 @@ struct src_lily_state {
     __device__ void load(const doc_rows & dr, int t, int col, float (&v)[4]) const {
         const int j0 = max(0, dr.lo - (t - k / 2)), j1 = min(k, dr.hi - (t - k / 2));
         float acc[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+        if (k <= TAPS_HOIST) {
+            // every tap's rows loaded first (clamped into the batch), then the fmas of taps j0..j1-1
+            v4f w[TAPS_HOIST], av[TAPS_HOIST], xv[TAPS_HOIST];
+#pragma unroll
+            for (int j = 0; j < TAPS_HOIST; ++j) {
+                if (j >= k) break;
+                const size_t o = (size_t) min(max(t + j - k / 2, 0), T - 1) * C + col;
+                w[j] = *reinterpret_cast<const v4f *>(taps + (size_t) j * C + col);
+                av[j] = *reinterpret_cast<const v4f *>(a + o);
+                xv[j] = *reinterpret_cast<const v4f *>(x + o);
+            }
+#pragma unroll
+            for (int j = 0; j < TAPS_HOIST; ++j) {
+                if (j >= k || j < j0 || j >= j1) continue;
+                acc[0] = __builtin_fmaf(w[j].x, av[j].x * xv[j].x, acc[0]);
+                acc[1] = __builtin_fmaf(w[j].y, av[j].y * xv[j].y, acc[1]);
+                acc[2] = __builtin_fmaf(w[j].z, av[j].z * xv[j].z, acc[2]);
+                acc[3] = __builtin_fmaf(w[j].w, av[j].w * xv[j].w, acc[3]);
+            }
+            const v4f bv = *reinterpret_cast<const v4f *>(b + (size_t) t * C + col);
+            v[0] = acc[0] * bv.x; v[1] = acc[1] * bv.y; v[2] = acc[2] * bv.z; v[3] = acc[3] * bv.w;
+            return;
+        }
         for (int j = j0; j < j1; ++j) {
             const size_t o = (size_t) (t + j - k / 2) * C + col;
             const v4f w = *reinterpret_cast<const v4f *>(taps + (size_t) j * C + col);
@@ -708,8 +729,8 @@ __device__ __forceinline__ v4i bload16(__amdgpu_buffer_rsrc_t r, uint32_t voff, 
 // src_lily_state for k <= TAPS_HOIST with the products a * x of a workgroup's 16 rows and their
 // neighbours formed once, in LDS: tap j of row t reads row t + j - k / 2 there. Loading them per
 // tap read a and x k times over through the caches; now 1.25 times. The rows' documents, b and
-// the products' inputs are all fetched before the one barrier. 33,000 rows of 1,024 124 -> 115 us,
-// 435 MB at 3.8 TB/s (a device copy 5.5).
+// the products' inputs are all fetched before the one barrier. For launches of many rows: 33,000
+// of 1,024 124 -> 115 us, 435 MB at 3.8 TB/s (a device copy 5.5).
 template <int ACT_MAX>
 __global__ __launch_bounds__(256) void lily_state_quantize_kernel(src_lily_state src, int T, int n_in, int KS, int n_blk,
                                                                   int8_t * __restrict__ q, float * __restrict__ sx) {
@@ -3805,7 +3826,10 @@ static int32_t launch_produce(const char * what, const Src & src, int32_t T, int
     const dim3 grid((unsigned) n_wg);
     hipStream_t s = (hipStream_t) stream;
     if constexpr (std::is_same_v<Src, src_lily_state>) {
-        if (src.k <= TAPS_HOIST) {             // the products of the taps' rows fit the kernel's LDS
+        // the products of the taps' rows fit the kernel's LDS; its barrier is dear to a launch of few
+        // rows (1,024 rows of 1,024: 12.2 us, 10.0 without; 8,192 rows 33.0 and 32.5; 33,000
+        // rows 115 and 124; 65,536 rows 204 and 222)
+        if (src.k <= TAPS_HOIST && n_wg >= 16LL * device_cus()) {
             if (act_max == 127) lily_state_quantize_kernel<127><<<grid, 256, 0, s>>>(src, T, n_in, d.KS, d.n_blk, q, sx);
             else                lily_state_quantize_kernel<63><<<grid, 256, 0, s>>>(src, T, n_in, d.KS, d.n_blk, q, sx);
             return launch_check(what);
