@@ -200,11 +200,11 @@ NXG_API int32_t nxg_attention(const float * q, const float * k, const float * v,
 
 /* op_attention (src/nexterabert.cpp:785-852) as nxg_attention, with a device workspace for
  * launches whose scores do not fit in LDS (more than ~2,400 keys per query with
- * n_head / n_kv_head dividing 16), or fit with room for one workgroup per CU (more than ~1,200
+ * n_head / n_kv_head dividing 16), or fit with room for one workgroup per CU (more than ~1,100
  * keys), or for two in a launch of more than 4 x the CUs' workgroups (e.g. 2 x 1,024 keys):
  * each score is computed once and kept in the workspace for the softmax and the values,
  * instead of kept in LDS or recomputed in each of three passes; the outputs are the same bits.
- * The workspace holds one slot of 16 * max_keys floats per resident workgroup; a smaller one
+ * The workspace holds two slots of 16 * max_keys floats per resident workgroup; a smaller one
  * (at least one slot) runs fewer workgroups at a time, and none (NULL, 0) the LDS kernel where
  * its scores fit, else the recomputing kernel. Other launches ignore it.
  * Calls that share a workspace must not overlap.
@@ -241,7 +241,7 @@ NXG_API int32_t nxg_upload_words(const void * src, int32_t n, void * dst, void *
 
 /* Sizing for nxg_attention_ws (no counterpart in the reference, whose op_attention keeps a
  * document's scores in host memory): the workspace it uses for these sizes: 0 when the launch does not need one,
- * else one slot per resident workgroup (a negative NXG_E* code for invalid sizes). */
+ * else two slots per resident workgroup (a negative NXG_E* code for invalid sizes). */
 NXG_API int64_t nxg_attention_workspace_bytes(int32_t T, int32_t n_head, int32_t n_kv_head, int32_t max_keys);
 
 /* op_qk_prep (src/nexterabert.cpp:590-632): the separable DyT (beta * tanh(alpha * x), with
