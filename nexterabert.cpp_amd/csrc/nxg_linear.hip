@@ -967,9 +967,10 @@ __device__ __forceinline__ bool finite4(const v4f & x) {
 //   values   register r, times 1 / sum, is the MFMA's A operand of keys 4r .. 4r + 3; the waves
 //            take 16 of the 64 dimensions each, all tiles
 // A tile is clean when every active pair attends to all its keys, none of them a pair's first or
-// in its last n % 8; others compute both trees and mask. Keys outside a pair's range get e = -0
-// (its products with finite values leave acc as it is); where an output is Inf or NaN the keys are
-// taken again one by one, each result kept only for the pairs that attend to the key.
+// in its last n % 8; others compute both trees and mask. Keys outside a pair's range get e = -0:
+// its products with finite values are zeros, which leave every acc but -0 as it is. Where an output
+// is Inf, NaN or a +0 that may stand for -0, the keys are taken again one by one, each result kept
+// only for the pairs that attend to the key.
 // Key and value rows come straight from memory (each is read once per workgroup) by buffer
 // loads that return 0 past the last key, whole lines to a few lanes, and turn into operand order
 // through a little LDS of the wave's own: a load whose neighbouring lanes are on different lines
@@ -1549,14 +1550,28 @@ __global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_pa
                     part(lds_tag{}, nt);
                 }
                 // an Inf or NaN value makes every pair's sum of its dimension Inf or NaN, whatever the
-                // weights, also for pairs that do not attend to it: key by key then
+                // weights, also for pairs that do not attend to it: key by key then. A key past a pair's
+                // last turns a sum of -0 (every product underflowed) into +0 where its value is negative:
+                // a +0 is taken again too, unless the pair's last value is +0, which makes it one
 #pragma unroll
                 for (int u = 0; u < NP; ++u) {
                     const uint32_t rows = (uint32_t) __ballot(act[u]) & 0xffffu;
                     auto is_act = [&](int r) { return ((rows >> (4 * g4 + r)) & 1) != 0; };
+                    constexpr int INF_NAN = 0x207, PLUS_ZERO = 0x40;
                     bool bad = false;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) bad = bad || (is_act(r) && !__builtin_isfinite(acc[u][r]));
+                    for (int r = 0; r < 4; ++r) bad = bad || (is_act(r) && __builtin_amdgcn_classf(acc[u][r], INF_NAN | PLUS_ZERO));
+                    if (__any(bad)) {
+                        bad = false;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int j = __shfl(hi[u], 4 * g4 + r) - 1 - kl;
+                            const uint32_t last = __builtin_amdgcn_raw_buffer_load_b32(
+                                vr, (int) ((uint32_t) j * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0);
+                            bad = bad || (is_act(r) && (__builtin_amdgcn_classf(acc[u][r], INF_NAN) ||
+                                                        (__builtin_amdgcn_classf(acc[u][r], PLUS_ZERO) && last != 0)));
+                        }
+                    }
                     if (__any(bad)) {
                         acc[u] = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll 1

@@ -2,7 +2,7 @@
 wrong: key counts around the 16-key tile and the 8-key group, every head ratio that divides 16,
 bands narrower and wider than a tile, workgroups whose queries lie in several documents (also
 where those documents' scores do not fit together), scores split between LDS and a workspace of
-any size and alignment, and non-finite queries, keys and values."""
+any size and alignment, non-finite queries, keys and values, and sums that underflow to -0."""
 from __future__ import annotations
 
 import numpy as np
@@ -44,6 +44,7 @@ def check(nxg, orc, torch, lengths, half, H, G, workspaces=(None,), seed=0, spoi
         print(f"attention lengths={lengths} half={half} H={H} G={G} workspace={size}", flush=True)
         y = nxg.attention(*dev, cu, scale, H, G, half, workspace=ws).cpu().numpy()
         assert ((bits(y) == bits(ref)) | (np.isnan(y) & np.isnan(ref))).all()
+    return ref
 
 
 @pytest.mark.parametrize("H,G", [(4, 4), (4, 2), (4, 1), (8, 1), (16, 1)])
@@ -90,3 +91,26 @@ def test_non_finite_queries_keys_values(nxg, orc, torch, dev, half):
     def tiny(q, k, v):
         v *= np.float32(1e-38)            # sums among the subnormals
     check(nxg, orc, torch, n, half, 8, 2, seed=4, spoil=tiny)
+
+
+@pytest.mark.parametrize("lengths,half,workspace", [
+    ([5, 40, 24, 2, 300], -1, None),      # documents that share a workgroup, padding after the last
+    ([5, 40, 24, 2, 300], 9, None),       # keys past the band
+    ([100, 2900, 60], -1, "auto"),
+    ([2900], 1300, "auto"),
+])
+def test_sums_that_underflow_keep_their_sign(nxg, orc, torch, dev, lengths, half, workspace):
+    """Products of the smallest subnormal with weights under one half round to -0 or +0 by the
+    value's sign: a sum of -0 stays -0 whatever the values of the keys that follow it outside the
+    pair's range, and +0 stays +0."""
+    def spoil(q, k, v):
+        rng = np.random.default_rng(5)
+        v[:] = np.float32(-1e-45)
+        v[:, :, 1] = np.float32(1e-45)
+        v[:, :, 2] = rng.choice(np.array([-1e-45, 1e-45, -0.0, 0.0], np.float32), v.shape[:2])
+        v[:, :, 3] = 0.0
+        v[:, :, 4] = -0.0
+        v[:, ::3, 5:20] = rng.standard_normal(v[:, ::3, 5:20].shape)
+        q *= np.float32(0.01)             # weights near 1 / n
+    ref = check(nxg, orc, torch, lengths, half, 4, 2, workspaces=(workspace,), seed=7, spoil=spoil)
+    assert (bits(ref) == 0x80000000).mean() > 0.3 and (bits(ref) == 0).any()
