@@ -1669,7 +1669,8 @@ constexpr int ATT_KS = 68;     // floats per staged row
 //   pass 3  w = e * (1 / sum) per key through LDS, then thread (dim d, 4 pairs) acc = fma(w,
 //           v[d], acc) over the keys in order: a tile's weights are read once per lane and
 //           broadcast per key by DPP row_newbcast (keys outside a pair's range with weight 0), or
-//           by readlane with a per-key range test on tiles with an Inf or NaN value
+//           by readlane with a per-key range test on tiles with an Inf or NaN value and on partial
+//           tiles that leave a +0, which may stand for -0
 // Keys and values are staged ATT_KT at a time ([key][ATT_KS]).
 __global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
     __shared__ __attribute__((aligned(16))) float tile[ATT_KT * ATT_KS];
@@ -1807,13 +1808,17 @@ __global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
 
     // pass 3: the weights, then the values
     const int d = tid & 63, pg = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int vlo[4], vn[4];
+    int vlo[4], vn[4], all_lo = INT_MIN, all_hi = INT_MAX;   // keys [all_lo, all_hi): every pair's
     float acc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int n = hi_s[4 * pg + i] - lo_s[4 * pg + i];
         vlo[i] = __builtin_amdgcn_readfirstlane(lo_s[4 * pg + i]);
         vn[i] = __builtin_amdgcn_readfirstlane(n <= p.max_keys ? n : 0);
+        if (vn[i] > 0) {
+            all_lo = max(all_lo, vlo[i]);
+            all_hi = min(all_hi, vlo[i] + vn[i]);
+        }
         acc[i] = 0.0f;
     }
     // a staged value tile holding a non-finite value (by tile parity): without one, a partial tile
@@ -1846,7 +1851,7 @@ __global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
         const int jn = min(ATT_KT, kh - j0);
         // pair i's weights of the tile: lane l holds key j0 + l (l < 32), broadcast per key
         int a[4], b[4];
-        const bool full = vbad_s[par] == 0;
+        bool by_key = vbad_s[par] != 0;
         float w0[4], w1[4];                                // keys j0 + k, j0 + 16 + k in lane k of each row
 #pragma unroll
         for (int i = 0; i < 4; ++i) {                      // keys [a, b) of the tile are pair i's
@@ -1858,13 +1863,29 @@ __global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
         auto wk = [&](int i, int jj) {
             return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(jj < 16 ? w0[i] : w1[i]), jj & 15));
         };
-        if (full) {
+        auto broadcast = [&]() {
             float vt[ATT_KT];
 #pragma unroll
             for (int jj = 0; jj < ATT_KT; ++jj) vt[jj] = tile[jj * ATT_KS + d];
             fmac_bcast4_16(acc, w0, vt);
             fmac_bcast4_16(acc, w1, vt + 16);
-        } else {
+        };
+        if (!by_key && j0 >= all_lo && j0 + ATT_KT <= all_hi) {
+            broadcast();
+        } else if (!by_key) {
+            // a product of weight 0 leaves every acc but -0 as it is, which it may turn into +0
+            const float was[4] = { acc[0], acc[1], acc[2], acc[3] };
+            broadcast();
+            bool zero = false;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) zero = zero || __float_as_uint(acc[i]) == 0;
+            by_key = __any(zero);
+            if (by_key) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = was[i];
+            }
+        }
+        if (by_key) {
             for (int jj = 0; jj < jn; ++jj) {
                 const float v = tile[jj * ATT_KS + d];
 #pragma unroll

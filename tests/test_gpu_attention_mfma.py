@@ -98,6 +98,8 @@ def test_non_finite_queries_keys_values(nxg, orc, torch, dev, half):
     ([5, 40, 24, 2, 300], 9, None),       # keys past the band
     ([100, 2900, 60], -1, "auto"),
     ([2900], 1300, "auto"),
+    ([100, 2900, 60], -1, None),          # attention_long_kernel
+    ([2900], 1300, None),
 ])
 def test_sums_that_underflow_keep_their_sign(nxg, orc, torch, dev, lengths, half, workspace):
     """Products of the smallest subnormal with weights under one half round to -0 or +0 by the
