@@ -495,7 +495,11 @@ __global__ __launch_bounds__(256) void rmsnorm_q8_kernel(const float * __restric
 // upper bound); n = x * log2(e) rounded to the nearest integer (ties to even); the
 // argument reduced in two fused steps, r = x - n * 0.693359375 - n * (-2.12194440e-4);
 // the degree-5 Cephes polynomial in r by fused Horner steps, completed as p * r^2 + (r + 1);
-// scaled by 2^n built in the exponent field ((n + 127) << 23).
+// scaled by 2^n. The reference multiplies by 2^n built in the exponent field, (n + 127) << 23 with n in
+// [-126, 127]; the results are normal numbers (p > 1.03 at n = -126, p < 1.42 at 127), so ldexp gives
+// the same bits in two instructions fewer (1,024 keys 66.3 -> 64.8 us in attention_mfma_kernel).
+// EXPONENT: the reference's form, faster in attention_long_kernel (8,192 keys 12.99 -> 12.72 ms).
+template <bool EXPONENT = false>
 __device__ __forceinline__ float exp_cephes(float x) {
     constexpr float P[6] = { 1.9875691500e-4f, 1.3981999507e-3f, 8.3334519073e-3f,
                              4.1665795894e-2f, 1.6666665459e-1f, 5.0000001201e-1f };
@@ -508,6 +512,7 @@ __device__ __forceinline__ float exp_cephes(float x) {
 #pragma unroll
     for (int i = 1; i < 6; ++i) p = __builtin_fmaf(p, r, P[i]);
     p = __builtin_fmaf(p, r2, r + 1.0f);
+    if constexpr (EXPONENT) return p * __uint_as_float((uint32_t) ((int) n + 127) << 23);
     return __builtin_ldexpf(p, (int) n);
 }
 
@@ -1779,7 +1784,7 @@ __global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
                 const int kt = sk + 16 * r, jr = j0 + kt - plo;
                 if (!valid || jr < 0 || jr >= n_p) continue;
                 const float s = score_d64(qv, tile + kt * ATT_KS, jr < ng_p) * scale;
-                if (jr < ng_p) E[sp][kt] = exp_cephes(s - m);
+                if (jr < ng_p) E[sp][kt] = exp_cephes<true>(s - m);
                 else tail_e[sp][jr - ng_p] = expf_libm(s - m);
             }
             __syncthreads();
@@ -1841,7 +1846,7 @@ __global__ __launch_bounds__(256) void attention_long_kernel(attn_params p) {
                 continue;
             }
             const float s = score_d64(qv, tile + kt * ATT_KS, jr < ng_p) * scale;
-            E[sp][kt] = (jr < ng_p ? exp_cephes(s - m) : expf_libm(s - m)) * inv;
+            E[sp][kt] = (jr < ng_p ? exp_cephes<true>(s - m) : expf_libm(s - m)) * inv;
         }
         __syncthreads();                                   // the keys have been read
         stage();
