@@ -974,8 +974,8 @@ __device__ __forceinline__ bool finite4(const v4f & x) {
 // A tile is clean when every active pair attends to all its keys, none of them a pair's first or
 // in its last n % 8; others compute both trees and mask. Keys outside a pair's range get e = -0:
 // its products with finite values are zeros, which leave every acc but -0 as it is. Where an output
-// is Inf, NaN or a +0 that may stand for -0, the keys are taken again one by one, each result kept
-// only for the pairs that attend to the key.
+// is Inf, NaN or a +0 that may stand for -0, the values are taken again: clean tiles as they were,
+// the others' keys one by one, each result kept only for the pairs that attend to the key.
 // Key and value rows come straight from memory (each is read once per workgroup) by buffer
 // loads that return 0 past the last key, whole lines to a few lanes, and turn into operand order
 // through a little LDS of the wave's own: a load whose neighbouring lanes are on different lines
@@ -1555,9 +1555,11 @@ __global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_pa
                     part(lds_tag{}, nt);
                 }
                 // an Inf or NaN value makes every pair's sum of its dimension Inf or NaN, whatever the
-                // weights, also for pairs that do not attend to it: key by key then. A key past a pair's
-                // last turns a sum of -0 (every product underflowed) into +0 where its value is negative:
-                // a +0 is taken again too, unless the pair's last value is +0, which makes it one
+                // weights, also for pairs that do not attend to it: all again then, the tiles that are not
+                // clean key by key (all tiles so took 4,096 keys with one NaN row from 1.0 to 13.8 ms). A
+                // key past a pair's last turns a sum of -0 (every product underflowed) into +0 where its
+                // value is negative: a +0 is taken again too, unless the pair's last value is +0, which
+                // makes it one
 #pragma unroll
                 for (int u = 0; u < NP; ++u) {
                     const uint32_t rows = (uint32_t) __ballot(act[u]) & 0xffffu;
@@ -1580,18 +1582,41 @@ __global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_pa
                     if (__any(bad)) {
                         acc[u] = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll 1
-                        for (int j = 0; j < ATT_TILE * nt; ++j) {
-                            const v4f e = s_load(j / ATT_TILE, u, lx) * inv[u];
-                            const int r = (j & 15) >> 2;
-                            const bool mine = (j & 3) == g4;
-                            const float wj = r < 2 ? (r == 0 ? e.x : e.y) : (r == 2 ? e.z : e.w);
-                            const float vj = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                                vr, (int) ((uint32_t) j * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0));
-                            const v4f one = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? wj : 0.0f, mine ? vj : -0.0f, acc[u], 0, 0, 0);
-                            const uint64_t in = __ballot(act[u] && kl + j >= lo[u] && kl + j < hi[u]);
+                        for (int i0 = 0; i0 < nt; i0 += ATT_VC) {
+                            v4f wt[ATT_VC], vt[ATT_VC];
 #pragma unroll
-                            for (int k = 0; k < 4; ++k)
-                                if ((in >> (4 * g4 + k)) & 1) acc[u][k] = one[k];
+                            for (int k = 0; k < ATT_VC; ++k) {
+                                wt[k] = s_load(min(i0 + k, nt - 1), u, lx);
+#pragma unroll
+                                for (int r = 0; r < 4; ++r)
+                                    vt[k][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                        vr, (int) ((uint32_t) (ATT_TILE * (i0 + k) + 4 * r + g4) * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0));
+                            }
+                            keep_order();
+#pragma unroll
+                            for (int k = 0; k < ATT_VC; ++k) {
+                                const int i = i0 + k;
+                                if (i >= nt) break;
+                                wt[k] = wt[k] * inv[u];
+                                if (i >= c0 && i < c1) {   // every pair attends to every key
+#pragma unroll
+                                    for (int r = 0; r < 4; ++r)
+                                        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[k][r], vt[k][r], acc[u], 0, 0, 0);
+                                    continue;
+                                }
+#pragma unroll 1
+                                for (int j = 0; j < ATT_TILE; ++j) {
+                                    const int r = j >> 2, key = kl + ATT_TILE * i + j;
+                                    const bool mine = (j & 3) == g4;
+                                    const float wj = r < 2 ? (r == 0 ? wt[k].x : wt[k].y) : (r == 2 ? wt[k].z : wt[k].w);
+                                    const float vj = r < 2 ? (r == 0 ? vt[k].x : vt[k].y) : (r == 2 ? vt[k].z : vt[k].w);
+                                    const v4f one = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? wj : 0.0f, mine ? vj : -0.0f, acc[u], 0, 0, 0);
+                                    const uint64_t in = __ballot(act[u] && key >= lo[u] && key < hi[u]);
+#pragma unroll
+                                    for (int c = 0; c < 4; ++c)
+                                        if ((in >> (4 * g4 + c)) & 1) acc[u][c] = one[c];
+                                }
+                            }
                         }
                     }
 #pragma unroll

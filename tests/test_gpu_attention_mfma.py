@@ -116,3 +116,51 @@ def test_sums_that_underflow_keep_their_sign(nxg, orc, torch, dev, lengths, half
         q *= np.float32(0.01)             # weights near 1 / n
     ref = check(nxg, orc, torch, lengths, half, 4, 2, workspaces=(workspace,), seed=7, spoil=spoil)
     assert (bits(ref) == 0x80000000).mean() > 0.3 and (bits(ref) == 0).any()
+
+
+@pytest.mark.parametrize("lengths,half,workspaces", [
+    ([500, 70], -1, (None,)),
+    ([700], 200, (None,)),
+    ([40, 2900, 25], -1, ("auto", 16 * 2900 * 4)),
+    ([3000], 1300, ("auto", 16 * 2601 * 4)),
+])
+def test_non_finite_values_in_whole_and_partial_tiles(nxg, orc, torch, dev, lengths, half, workspaces):
+    """Inf and NaN values in tiles that every pair attends to and in the first, last and masked
+    ones: sums taken again give the oracle's bits, also those of the dimensions beside them."""
+    def spoil(q, k, v):
+        T = v.shape[1]
+        for j, x in ((0, np.inf), (17, np.nan), (T // 2, -np.inf), (T // 2 + 40, np.inf), (T - 1, np.nan)):
+            v[:, j, [j % 64, (j + 1) % 64]] = x
+        v[:, T // 3] = 3e38               # sums that overflow
+    ws = [w if isinstance(w, (str, type(None))) else torch.empty(w, dtype=torch.uint8, device="cuda") for w in workspaces]
+    ref = check(nxg, orc, torch, lengths, half, 2, 1, workspaces=ws, seed=11, spoil=spoil)
+    assert np.isfinite(ref).any() and not np.isfinite(ref).all()
+
+
+@pytest.mark.parametrize("n", [1024, 4096])
+def test_non_finite_values_cost_little(nxg, torch, dev, n):
+    """One NaN row makes every output NaN and every sum is taken again: about a third of the work,
+    not key by key (5 and 13 times the whole)."""
+    g = torch.Generator("cuda").manual_seed(n)
+    q = torch.randn(n, 1024, device="cuda", generator=g)
+    k, v = (torch.randn(8, n, 64, device="cuda", generator=g) for _ in range(2))
+    bad = v.clone()
+    bad[:, n // 3] = float("nan")
+    cu, scale = [0, n], np.array([0.1], np.float32)
+
+    def us(values):
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                y = nxg.attention(q, k, values, cu, scale, 16, 8, workspace="auto")
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 100)
+        return best, y
+
+    (fine, y), (nan, y_nan) = us(v), us(bad)
+    print(f"{n} keys: {fine:.0f} us, with a NaN row {nan:.0f}", flush=True)
+    assert torch.isfinite(y).all() and torch.isnan(y_nan).all()
+    assert nan < 3 * fine
