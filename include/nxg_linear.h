@@ -205,8 +205,9 @@ NXG_API int32_t nxg_attention(const float * q, const float * k, const float * v,
  * each score is computed once and kept in the workspace for the softmax and the values,
  * instead of kept in LDS or recomputed in each of three passes; the outputs are the same bits.
  * The workspace holds two slots of 16 * max_keys floats per resident workgroup; a smaller one
- * (at least one slot) runs fewer workgroups at a time, and none (NULL, 0) the LDS kernel where
- * its scores fit, else the recomputing kernel. Other launches ignore it.
+ * (at least one slot) runs fewer workgroups at a time, and one of less than a slot, or none
+ * (NULL, 0), the LDS kernel where its scores fit, else the recomputing kernel. Other launches
+ * ignore it.
  * Calls that share a workspace must not overlap.
  *   workspace        device memory, 4-byte aligned, or NULL
  *   workspace_bytes  its size (nxg_attention_workspace_bytes gives the size for every slot) */

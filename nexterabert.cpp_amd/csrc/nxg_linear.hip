@@ -4285,7 +4285,9 @@ int32_t nxg_attention_ws(const float * q, const float * k, const float * v, cons
     const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
     if (pl.kind != 2) {
         hipStream_t s = (hipStream_t) stream;
-        if (pl.kind == 1 && pl.need > 0) {
+        // less than one slot of all a group's scores is as no workspace: the few tiles past LDS may fit it,
+        // but only for a workgroup or two at a time (2,048 keys 91 ms with 1 KiB, 0.33 without)
+        if (pl.kind == 1 && pl.need > 0 && workspace_bytes >= pl.group_bytes) {
             // as many slots as the workspace holds, up to the resident workgroups: of two groups,
             // or of one where it holds none of two
             for (int np = 2; np >= 1; --np) {

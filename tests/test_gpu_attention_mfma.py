@@ -68,6 +68,19 @@ def test_scores_in_lds_and_workspace(nxg, orc, torch, dev, lengths, half, H, G):
     check(nxg, orc, torch, lengths, half, H, G, workspaces=(None, "auto", odd, one), seed=T)
 
 
+@pytest.mark.parametrize("n", [1536, 3000])
+def test_workspace_of_less_than_a_slot_is_not_used(nxg, orc, torch, dev, n):
+    """16 * max_keys floats are the least that is used; with less the launch is the one without a
+    workspace, its scores in LDS (1,536 keys) or recomputed (3,000), on the whole device."""
+    slot = 16 * n * 4
+    ws = [torch.full((b,), 0xA5, dtype=torch.uint8, device="cuda") for b in (1024, 4096, slot // 2, slot - 4, slot)]
+    check(nxg, orc, torch, [n], -1, 2, 1, workspaces=[None] + ws, seed=n)
+    for w in ws[:-1]:
+        assert bool((w == 0xA5).all()), f"{w.numel()} bytes were written"
+    if n == 3000:                         # (a workgroup by itself keeps 1,536 keys in LDS)
+        assert not bool((ws[-1] == 0xA5).all())
+
+
 @pytest.mark.parametrize("half", [-1, 9])
 def test_non_finite_queries_keys_values(nxg, orc, torch, dev, half):
     n = [40, 70, 21]
