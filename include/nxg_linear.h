@@ -207,7 +207,7 @@ NXG_API int32_t nxg_attention(const float * q, const float * k, const float * v,
  * The workspace holds two slots of 16 * max_keys floats per resident workgroup; a smaller one
  * (at least one slot) runs fewer workgroups at a time, and one of less than a slot, or none
  * (NULL, 0), the LDS kernel where its scores fit, else the recomputing kernel. Other launches
- * ignore it.
+ * ignore it, and so do those of more than 2^23 keys (the recomputing kernel).
  * Calls that share a workspace must not overlap.
  *   workspace        device memory, 4-byte aligned, or NULL
  *   workspace_bytes  its size (nxg_attention_workspace_bytes gives the size for every slot) */
@@ -242,7 +242,8 @@ NXG_API int32_t nxg_upload_words(const void * src, int32_t n, void * dst, void *
 
 /* Sizing for nxg_attention_ws (no counterpart in the reference, whose op_attention keeps a
  * document's scores in host memory): the workspace it uses for these sizes: 0 when the launch does not need one,
- * else two slots per resident workgroup (a negative NXG_E* code for invalid sizes). */
+ * or would not use one (more than 2^23 keys, which are always recomputed), else two slots per
+ * resident workgroup (a negative NXG_E* code for invalid sizes). */
 NXG_API int64_t nxg_attention_workspace_bytes(int32_t T, int32_t n_head, int32_t n_kv_head, int32_t max_keys);
 
 /* op_qk_prep (src/nexterabert.cpp:590-632): the separable DyT (beta * tanh(alpha * x), with

@@ -4208,7 +4208,7 @@ int64_t nxg_attention_workspace_bytes(int32_t T, int32_t n_head, int32_t n_kv_he
     int rc = check_device();
     if (rc) return rc;
     const attn_plan pl = plan_attention(T, n_head, n_kv_head, max_keys);
-    if (pl.kind != 1) return 0;
+    if (pl.kind != 1 || pl.need == 0) return 0;            // need 0: more than ATT_MAX_KEYS keys
     return std::min(pl.n_groups, 2 * attention_slots()) * pl.group_bytes;
 }
 

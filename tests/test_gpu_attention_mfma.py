@@ -81,6 +81,28 @@ def test_workspace_of_less_than_a_slot_is_not_used(nxg, orc, torch, dev, n):
         assert not bool((ws[-1] == 0xA5).all())
 
 
+def test_workspace_asked_for_is_one_that_is_used(nxg, orc, torch, dev):
+    """Past 2^23 keys the scores are recomputed whatever the workspace: none is asked for (a slot for
+    every workgroup would be 550 GB), and a call under such a bound runs without one."""
+    at, past = 1 << 23, (1 << 23) + 1
+    full = nxg.attention_workspace_bytes(past, 16, 8, at)
+    assert full > 0 and full % (64 * at) == 0
+    assert nxg.attention_workspace_bytes(past, 16, 8, past) == 0
+    H, G, T = 2, 1, 40
+    rng = np.random.default_rng(2)
+    q = rng.standard_normal((T, H * 64)).astype(np.float32)
+    k, v = (rng.standard_normal((G, T, 64)).astype(np.float32) for _ in range(2))
+    d = [torch.from_numpy(a).cuda() for a in (q, k, v)]
+    cu, sc = torch.tensor([0, T], dtype=torch.int32, device="cuda"), torch.full((1,), 0.125, device="cuda")
+    ws, out = torch.full((4096,), 0xA5, dtype=torch.uint8, device="cuda"), torch.empty_like(d[0])
+    L = nxg.load_library()
+    args = [t.data_ptr() for t in (*d, cu)] + [1, sc.data_ptr(), T, H, G, -1, past, out.data_ptr()]
+    assert L.nxg_attention_ws(*args, ws.data_ptr(), ws.numel(), None) == 0
+    torch.cuda.synchronize()
+    assert bool((ws == 0xA5).all())
+    assert (bits(out.cpu().numpy()) == bits(orc.attention(q, k, v, [0, T], np.float32([0.125]), H, G))).all()
+
+
 @pytest.mark.parametrize("half", [-1, 9])
 def test_non_finite_queries_keys_values(nxg, orc, torch, dev, half):
     n = [40, 70, 21]
