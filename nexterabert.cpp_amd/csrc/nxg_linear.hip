@@ -734,8 +734,8 @@ __device__ __forceinline__ v4i bload16(__amdgpu_buffer_rsrc_t r, uint32_t voff, 
 // src_lily_state for k <= TAPS_HOIST with the products a * x of a workgroup's 16 rows and their
 // neighbours formed once, in LDS: tap j of row t reads row t + j - k / 2 there. Loading them per
 // tap read a and x k times over through the caches; now 1.25 times. The rows' documents, b and
-// the products' inputs are all fetched before the one barrier. For launches of many rows: 33,000
-// of 1,024 124 -> 115 us, 435 MB at 3.8 TB/s (a device copy 5.5).
+// the products' inputs are all fetched before the one barrier. For inputs past the last-level cache:
+// 33,000 rows of 1,024 119 -> 108 us, 435 MB at 4.0 TB/s (a device copy 5.5).
 template <int ACT_MAX>
 __global__ __launch_bounds__(256) void lily_state_quantize_kernel(src_lily_state src, int T, int n_in, int KS, int n_blk,
                                                                   int8_t * __restrict__ q, float * __restrict__ sx) {
@@ -3892,10 +3892,12 @@ static int32_t launch_produce(const char * what, const Src & src, int32_t T, int
     const dim3 grid((unsigned) n_wg);
     hipStream_t s = (hipStream_t) stream;
     if constexpr (std::is_same_v<Src, src_lily_state>) {
-        // the products of the taps' rows fit the kernel's LDS; its barrier is dear to a launch of few
-        // rows (1,024 rows of 1,024: 12.2 us, 10.0 without; 8,192 rows 33.0 and 32.5; 33,000
-        // rows 115 and 124; 65,536 rows 204 and 222)
-        if (src.k <= TAPS_HOIST && n_wg >= 16LL * device_cus()) {
+        // the products of the taps' rows fit the kernel's LDS. Its saving is memory traffic, its cost a
+        // barrier: ahead where a, x and b are more than the 256 MiB last-level cache holds for the taps'
+        // repeated reads (rows of 1,024, per tap and here: 24,000 85 and 75 us, 22,000 74.7 and 69.5,
+        // 21,000 66.6 and 66.0, 20,000 57.1 and 63.6, 16,384 44 and 53; rows of 256: 89,000 76 and 74,
+        // 65,536 44 and 55)
+        if (src.k <= TAPS_HOIST && 3LL * T * n_in * (long long) sizeof(float) > 256LL << 20) {
             if (act_max == 127) lily_state_quantize_kernel<127><<<grid, 256, 0, s>>>(src, T, n_in, d.KS, d.n_blk, q, sx);
             else                lily_state_quantize_kernel<63><<<grid, 256, 0, s>>>(src, T, n_in, d.KS, d.n_blk, q, sx);
             return launch_check(what);

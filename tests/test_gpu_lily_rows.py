@@ -1,5 +1,5 @@
 """GPU: SnowLily's state over enough rows for the kernel that forms the a * x products in LDS
-(4,096 workgroups of 16 rows by 256 inputs on 256 CUs), bit for bit against the oracle: documents
+(a, x and b more than 256 MiB together) and over fewer, bit for bit against the oracle: documents
 that begin and end inside a 16-row group, even and odd kernels, inputs that are no multiple of
 256, non-finite values beside the documents' edges."""
 from __future__ import annotations
@@ -28,6 +28,11 @@ def dev(torch, nxg):
     (1024, 2, [16390]),
     (288, 3, [30000, 7, 1, 2762]),
     (96, 1, [65500, 9, 30]),
+    (1024, 5, [1, 2, 3, 15, 16, 17, 33, 5000, 16758]),      # 21,845 rows: just below 256 MiB
+    (1024, 5, [1, 2, 3, 15, 16, 17, 33, 5000, 16759]),      # just past, as all that follow
+    (1024, 2, [22001]),
+    (288, 3, [75000, 7, 1, 2762]),
+    (96, 1, [233000, 9, 30]),
 ])
 def test_lily_state_many_rows(nxg, orc, torch, dev, C, k, lengths):
     print(f"lily state C={C} k={k} lengths={lengths}", flush=True)
