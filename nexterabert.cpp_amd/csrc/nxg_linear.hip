@@ -4296,9 +4296,14 @@ int32_t nxg_attention_ws(const float * q, const float * k, const float * v, cons
                 const int lds_tiles = attention_ws_lds_tiles(np);
                 const int ws_tiles = std::max(attention_need(max_keys, rep, np) - lds_tiles, 1);
                 const long long n_wg_all = (long long) n_kv_head * ((T + np * ATT_P / rep - 1) / (np * ATT_P / rep));
-                const long long n_slots = std::min({n_wg_all, attention_slots(),
-                                                    (long long) (workspace_bytes / ((long long) ws_tiles * np * ATT_TILE_BYTES))});
+                long long n_slots = std::min({n_wg_all, attention_slots(),
+                                              (long long) (workspace_bytes / ((long long) ws_tiles * np * ATT_TILE_BYTES))});
                 if (n_slots < 1) continue;
+                // each workgroup has its share of the work from the start, so all wait for those that share a
+                // CU: one per CU unless half the CUs could have a second (8,192 keys of two groups: 258
+                // slots 8.10 ms, 322 6.41, 256 5.96, 387 5.58; 65,536 keys 258 slots 598 ms, 256 405)
+                const int cus = device_cus();
+                if (n_slots < n_wg_all && n_slots > cus && 2 * n_slots < 3LL * cus) n_slots = cus;
                 const dim3 grid((unsigned) n_slots), block(256);
                 const size_t lds = (size_t) lds_tiles * np * ATT_TILE_BYTES;
                 if (np == 2) attention_mfma_kernel<true, 2><<<grid, block, lds, s>>>(p, lds_tiles, ws_tiles, (float *) workspace);

@@ -81,6 +81,32 @@ def test_workspace_of_less_than_a_slot_is_not_used(nxg, orc, torch, dev, n):
         assert not bool((ws[-1] == 0xA5).all())
 
 
+def test_half_a_workspace_is_no_slower_than_less(nxg, torch, dev):
+    """Half the workspace holds slots for a workgroup on every CU and a few more, which would share
+    theirs and have all others wait: 1.3 times the time of 3/8 of the workspace."""
+    n = 8192
+    g = torch.Generator("cuda").manual_seed(n)
+    q = torch.randn(n, 1024, device="cuda", generator=g)
+    k, v = (torch.randn(8, n, 64, device="cuda", generator=g) for _ in range(2))
+    full = nxg.attention_workspace_bytes(n, 16, 8, n)
+
+    def ms(size):
+        ws, best = torch.empty(size, dtype=torch.uint8, device="cuda"), float("inf")
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            y = nxg.attention(q, k, v, [0, n], np.array([0.1], np.float32), 16, 8, workspace=ws)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best, y
+
+    (half, y_half), (less, y_less) = ms(full // 2), ms(full * 3 // 8)
+    print(f"{n} keys: half the workspace {half:.2f} ms, 3/8 {less:.2f}", flush=True)
+    assert torch.equal(y_half.view(torch.int32), y_less.view(torch.int32))
+    assert half < 1.1 * less
+
+
 def test_workspace_asked_for_is_one_that_is_used(nxg, orc, torch, dev):
     """Past 2^23 keys the scores are recomputed whatever the workspace: none is asked for (a slot for
     every workgroup would be 550 GB), and a call under such a bound runs without one."""
