@@ -225,3 +225,31 @@ def test_non_finite_values_cost_little(nxg, torch, dev, n):
     print(f"{n} keys: {fine:.0f} us, with a NaN row {nan:.0f}", flush=True)
     assert torch.isfinite(y).all() and torch.isnan(y_nan).all()
     assert nan < 3 * fine
+
+
+@pytest.mark.parametrize("workspace", ["auto", "slot"])
+@pytest.mark.parametrize("lengths,half", [([40, 2900, 21], -1), ([3100], 1400)])
+def test_non_finite_and_extreme_scores_in_the_workspace(nxg, orc, torch, dev, lengths, half, workspace):
+    """Scores that live in a workspace slot: the maximum and the sums of the slot's exponentials are
+    code of their own. NaN and Inf keys and queries in tiles kept in LDS, in the slot and among a
+    pair's last n % 8 keys, a NaN first key, and scores over +-400."""
+    T, most = sum(lengths), max(lengths) if half < 0 else min(max(lengths), 2 * half + 1)
+    start = lengths[0] if len(lengths) > 1 else 0             # of the long document
+    ws = (torch.empty(16 * most * 4, dtype=torch.uint8, device="cuda") if workspace == "slot" else "auto",)
+
+    def spoil_keys(rows):
+        def spoil(q, k, v):
+            for j, x in rows:
+                k[0, start + j, j % 64] = x
+            q[start + 1500, 5], q[start + 77, 70] = np.inf, np.nan
+        return spoil
+    end = lengths[1] if len(lengths) > 1 else lengths[0]
+    for rows in ([(0, np.nan)],                               # the first score of every pair, or of the first rows
+                 [(30, np.nan), (1000, np.inf), (2500, np.nan), (2600, -np.inf)],
+                 [(end - 1, np.nan), (end - 2, np.inf)]):     # the last keys
+        ref = check(nxg, orc, torch, lengths, half, 2, 1, workspaces=ws, seed=end, spoil=spoil_keys(rows))
+        assert np.isfinite(ref).any()
+
+    def extreme(q, k, v):
+        q *= 50
+    check(nxg, orc, torch, lengths, half, 2, 1, workspaces=ws, seed=3, spoil=extreme)
