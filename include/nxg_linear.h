@@ -235,7 +235,8 @@ NXG_API int32_t nxg_attention_noalloc(const float * q, const float * k, const fl
  * counterpart in the reference. For the small arrays that calls here take on the device
  * (document offsets, scales): the words are read before the call returns and travel as
  * launch arguments, 896 to a launch, where a copy from pageable memory would wait for the
- * stream's earlier work.
+ * stream's earlier work. Under graph capture the words of capture time are recorded, and every
+ * replay writes those.
  *   src  host memory   dst  device memory, 4-byte aligned   n  at most NXG_UPLOAD_MAX_WORDS */
 #define NXG_UPLOAD_MAX_WORDS 3584
 NXG_API int32_t nxg_upload_words(const void * src, int32_t n, void * dst, void * stream);

@@ -390,7 +390,9 @@ UPLOAD_MAX_WORDS = 3584                 # NXG_UPLOAD_MAX_WORDS
 def _uploaded(a, device):
     """A host array of 32-bit values as a device tensor, made on torch's current stream. Small ones go
     by nxg_upload_words, which does not wait for the stream (torch.tensor's copy from pageable
-    memory does: 3 of them cost a 512-token attention mixer about 50 of its 160 us)."""
+    memory does: 3 of them cost a 512-token attention mixer about 50 of its 160 us). Under graph
+    capture the values of capture time are recorded for every replay; larger arrays are refused
+    there, as that copy is: pass device tensors to change offsets or scales between replays."""
     torch = _torch()
     if a.ndim != 1 or a.size == 0 or a.size > UPLOAD_MAX_WORDS or device.index not in (None, _raw_device()):
         return torch.tensor(a, device=device)

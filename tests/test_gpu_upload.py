@@ -1,6 +1,6 @@
 """GPU: nxg_upload_words and the offsets and scales that go by it: sizes around a launch's 896
-words, past the largest (which takes torch's copy), and calls in a row whose host arrays are
-changed right after the call."""
+words, past the largest (which takes torch's copy), calls in a row whose host arrays are
+changed right after the call, and calls recorded in a graph."""
 from __future__ import annotations
 
 import numpy as np
@@ -39,3 +39,40 @@ def test_refused(nxg, torch):
     assert L.nxg_upload_words(None, 4, d.data_ptr(), None) == nxg.NXG_EINVAL
     assert L.nxg_upload_words(a.ctypes.data, 4, d.data_ptr() + 2, None) == nxg.NXG_EINVAL
     assert L.nxg_upload_words(None, 0, None, None) == nxg.NXG_OK
+
+
+def test_captured_calls_keep_the_words_of_capture_time(nxg, torch):
+    """Host offsets and scales of calls under graph capture: every replay uses those of capture time,
+    whatever happens to the arrays afterwards, with eager work of the same calls in between."""
+    nxg.init()
+    g = torch.Generator("cuda").manual_seed(4)
+    T, H, G = 150, 4, 2
+    new = lambda *shape: torch.randn(*shape, device="cuda", generator=g)
+    q, k, v, a, x, b, taps = new(T, H * 64), new(G, T, 64), new(G, T, 64), *(new(T, 64) for _ in range(3)), new(5, 64)
+    cu, scale = np.array([0, 40, 41, T], np.int32), np.array([0.1, 0.2, 0.3], np.float32)
+
+    def calls(cu, scale):
+        return nxg.attention(q, k, v, cu, scale, H, G), nxg.lily_state_quantize_rows(a, x, b, taps, cu)
+
+    def same(y, ref):
+        return torch.equal(y[0], ref[0]) and torch.equal(y[1].q, ref[1].q) and torch.equal(y[1].sx, ref[1].sx)
+    other = calls([0, T], np.array([0.4], np.float32))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        calls(cu, scale)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = calls(cu, scale)
+    kept = cu.copy(), scale.copy()
+    cu[1:3], scale[:] = (7, 90), 9.0
+    for rep in range(3):
+        q.normal_(generator=g)
+        graph.replay()
+        torch.cuda.synchronize()
+        print(f"captured offsets: replay {rep}", flush=True)
+        ref = calls(*kept)
+        assert same(y, ref) and not torch.equal(ref[0], other[0])
+        calls(cu, scale)
