@@ -1051,12 +1051,11 @@ __device__ __forceinline__ v4f bload16f(__amdgpu_buffer_rsrc_t r, uint32_t voff)
 // vector instructions do not hide under it (16 MFMAs with 2 or 8 vector instructions each on four
 // waves: 38.6 and 57 cycles per MFMA against 32.6), so a tile costs a SIMD at least 32 x 32 cycles
 // and ~140 vector instructions of ~2.5, about 1,400. The matrix cores take the operands' traffic
-// and issue slots away: the same FMAs as vector
-// instructions, with their LDS reads and broadcasts, ran at about 30 TFLOP/s; this runs at 45-65. At most 128
-// registers, so that four workgroups share a CU: two took 181 us where four take 161 (8 x 1,024
-// tokens, band 256). Kernel times: 1,024 keys 75 us, 8 x 1,024 tokens
-// in bands of 257 keys 161 us, 32 documents of 16 to 2,048 tokens 2.80 ms (on the vector unit
-// about 150, 250 us and 7.4 ms).
+// and issue slots away: the same FMAs as vector instructions, with their LDS reads and broadcasts,
+// ran at about 30 TFLOP/s; this runs at 45-65. At most 128 registers, so that four workgroups share
+// a CU (a form of 168-189 took 181 us where one of 125 took 161: 8 x 1,024 tokens, band 256). Calls:
+// 1,024 keys 65 us, 8 x 1,024 tokens in bands of 257 keys 138 us, 32 documents of 16 to 2,048
+// tokens 2.78 ms (on the vector unit 140, 241 us and 7.1 ms).
 // Lane numbers are taken anew in each phase: kept across them, the addresses made from them cost
 // 50 registers.
 template <bool WS, int NP>
@@ -1071,8 +1070,9 @@ __global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_pa
     const int lg_rep = __builtin_ctz((unsigned) (p.H / p.G)), rep = 1 << lg_rep, nq = PAIRS >> lg_rep;
     const int n_tiles = p.G * ((p.T + nq - 1) / nq);
     const int cap = ATT_TILE * (lds_tiles + ws_tiles);
-    // the wave that adds up: waves 0 of a CU's workgroups share a SIMD, so it goes by their slot
-    // there (hwreg HW_ID's wave slot, 4 bits at 0)
+    // the wave that adds up: waves 0 of a CU's workgroups share a SIMD, so it goes by their slot there
+    // (hwreg HW_ID's wave slot, 4 bits at 0). Little: 1,024 keys 65.0 us, always wave 0 65.4; even
+    // where the launch has more rounds
     __shared__ int adder_s;
     if (threadIdx.x == 0) adder_s = __builtin_amdgcn_s_getreg(4 | (0 << 6) | (3 << 11)) & 3;
     float * const slot = WS ? ws + (size_t) blockIdx.x * ws_tiles * (NP * ATT_TILE_BYTES / 4) : nullptr;

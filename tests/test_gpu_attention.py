@@ -2,8 +2,9 @@
 documents of 1 to 4,000 tokens (key counts off multiples of 8 send the last keys through
 hsum256 and the C library's expf), full and banded (swa) attention, 16 query / 8 KV heads,
 per-document scales, and scores large enough to underflow exp in both its forms. The kernel
-depends on the keys per query: the tile kernel up to ~2,400 (scores in LDS), the three-pass
-kernel beyond (scores recomputed), the row kernel for head ratios that do not divide 16."""
+depends on the keys per query: the matrix-core kernel with its scores in LDS up to ~2,400, in LDS
+and a workspace where one is given (from ~1,100 keys), the three-pass kernel (scores recomputed)
+past LDS without one; the row kernel for head ratios that do not divide 16."""
 from __future__ import annotations
 
 import numpy as np
@@ -77,7 +78,7 @@ def test_attention_long_document(nxg, orc, torch, dev):
 
 @pytest.mark.parametrize("lengths,half", [([4000], 1500), ([3000, 5, 700], -1)])
 def test_attention_long_documents(nxg, orc, torch, dev, lengths, half):
-    """Past the tile kernel's LDS: the three-pass kernel, banded and packed."""
+    """Past LDS without a workspace: the three-pass kernel, banded and packed."""
     say(f"attention long lengths={lengths} half={half}")
     rng = np.random.default_rng(len(lengths) + 3)
     H, G = 2, 1
@@ -93,9 +94,9 @@ def test_attention_long_documents(nxg, orc, torch, dev, lengths, half):
 @pytest.mark.parametrize("lengths,half,H,G", [([4000], 1500, 2, 1), ([3000, 5, 700], -1, 2, 1),
                                               ([2600, 1, 9], -1, 4, 2), ([2500], 1300, 1, 1)])
 def test_attention_stored_scores(nxg, orc, torch, dev, lengths, half, H, G):
-    """nxg_attention_ws past the tile kernel's LDS: the scores written once to the workspace and
-    read back by the softmax and the values give the oracle's bits, with a slot for every
-    resident workgroup and with 3 slots (each workgroup then takes many tiles in turn)."""
+    """nxg_attention_ws past LDS: the scores written once to LDS and the workspace and read back by
+    the softmax and the values give the oracle's bits, with slots for every resident workgroup and
+    with 3 (each workgroup then takes many groups of queries in turn)."""
     say(f"attention stored scores lengths={lengths} half={half} H={H} G={G}")
     rng = np.random.default_rng(len(lengths) + 11 * H + half)
     cu = nxg.cu_offsets_of(lengths)
@@ -117,8 +118,8 @@ def test_attention_stored_scores(nxg, orc, torch, dev, lengths, half, H, G):
 @pytest.mark.parametrize("lengths", [[1536], [1024, 1024], [1100, 900, 48]])
 def test_attention_stored_where_tiles_fit(nxg, orc, torch, dev, lengths):
     """Scores that fit in LDS with room for one workgroup per CU (1,536 keys), or for two in a
-    launch of more than two rounds (2,048 tiles), go to the stored kernel when a workspace is
-    given, to the tile kernel without one: both give the oracle's bits."""
+    launch of more than two rounds (2,048 groups of 16 pairs), go to LDS and the workspace when one
+    is given, to LDS alone without: both give the oracle's bits."""
     say(f"attention stored where tiles fit lengths={lengths}")
     rng = np.random.default_rng(sum(lengths) + 21)
     H, G = 16, 8
@@ -183,11 +184,11 @@ def test_attention_extreme_scores(nxg, orc, torch, dev):
                                                  ([3000], 1300, 2, 1, "auto"), ([40, 2900, 25], -1, 2, 1, "auto"),
                                                  ([40, 2900, 25], -1, 2, 1, None)])
 def test_attention_non_finite_values_outside_a_pair(nxg, orc, torch, dev, lengths, half, H, G, ws):
-    """Inf and NaN values at keys that other pairs of the same staged tile do not attend to (a
-    neighbour document, outside a band), on the tile, stored and recomputing kernels: value
-    tiles that hold them take the per-key path, the others the broadcast path with zero weights
-    outside a pair's keys; the pairs that do not see them stay finite and give the oracle's
-    bits, the others its NaN / Inf pattern."""
+    """Inf and NaN values at keys that other pairs of the same tile do not attend to (a neighbour
+    document, outside a band), with scores in LDS, in a workspace and recomputed: the matrix-core
+    kernel takes such sums again, their masked tiles key by key; the recomputing one takes the
+    value tiles that hold them key by key. The pairs that do not see them stay finite and give
+    the oracle's bits, the others its NaN / Inf pattern."""
     say(f"attention non-finite values lengths={lengths} half={half} H={H} G={G} ws={ws}")
     rng = np.random.default_rng(sum(lengths) + 31)
     cu = nxg.cu_offsets_of(lengths)
@@ -270,9 +271,8 @@ def test_head_major(nxg, torch, dev):
 
 def test_attention_workspace_16384_keys(nxg, torch, dev):
     """One 16,384-token document: nxg_attention_ws with a 3-slot workspace (few workgroups at a
-    time, each over many query tiles; 3 MiB of slots, so pass 2 stores the exponentials for pass
-    3) and with a slot per resident workgroup (512 MiB: pass 3 recomputes them) equals the
-    recomputing kernel (no workspace) bit for bit."""
+    time, each over many groups of queries) and with slots for every resident workgroup equals
+    the recomputing kernel (no workspace) bit for bit."""
     say("attention 16,384 keys: 3-slot and full workspaces vs recomputing kernel")
     H, G, T = 2, 1, 16384
     g = torch.Generator("cuda").manual_seed(16)
