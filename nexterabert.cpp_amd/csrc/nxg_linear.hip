@@ -1572,7 +1572,7 @@ __global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_pa
                         bad = false;
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
-                            const int j = __shfl(hi[u], 4 * g4 + r) - 1 - kl;
+                            const int j = max(__shfl(hi[u], 4 * g4 + r) - 1 - kl, 0);   // < 0: another document's pair
                             const uint32_t last = __builtin_amdgcn_raw_buffer_load_b32(
                                 vr, (int) ((uint32_t) j * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0);
                             bad = bad || (is_act(r) && (__builtin_amdgcn_classf(acc[u][r], INF_NAN) ||
