@@ -1560,14 +1560,17 @@ __global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_pa
                 // key past a pair's last turns a sum of -0 (every product underflowed) into +0 where its
                 // value is negative: a +0 is taken again too, unless the pair's last value is +0, which
                 // makes it one
+                uint32_t rows[NP];
+                bool again[NP], any = false;
+#pragma unroll
+                for (int u = 0; u < NP; ++u) rows[u] = (uint32_t) __ballot(act[u]) & 0xffffu;
+                auto is_act = [&](int u, int r) { return ((rows[u] >> (4 * g4 + r)) & 1) != 0; };
 #pragma unroll
                 for (int u = 0; u < NP; ++u) {
-                    const uint32_t rows = (uint32_t) __ballot(act[u]) & 0xffffu;
-                    auto is_act = [&](int r) { return ((rows >> (4 * g4 + r)) & 1) != 0; };
                     constexpr int INF_NAN = 0x207, PLUS_ZERO = 0x40;
                     bool bad = false;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) bad = bad || (is_act(r) && __builtin_amdgcn_classf(acc[u][r], INF_NAN | PLUS_ZERO));
+                    for (int r = 0; r < 4; ++r) bad = bad || (is_act(u, r) && __builtin_amdgcn_classf(acc[u][r], INF_NAN | PLUS_ZERO));
                     if (__any(bad)) {
                         bad = false;
 #pragma unroll
@@ -1575,41 +1578,54 @@ __global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_pa
                             const int j = max(__shfl(hi[u], 4 * g4 + r) - 1 - kl, 0);   // < 0: another document's pair
                             const uint32_t last = __builtin_amdgcn_raw_buffer_load_b32(
                                 vr, (int) ((uint32_t) j * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0);
-                            bad = bad || (is_act(r) && (__builtin_amdgcn_classf(acc[u][r], INF_NAN) ||
-                                                        (__builtin_amdgcn_classf(acc[u][r], PLUS_ZERO) && last != 0)));
+                            bad = bad || (is_act(u, r) && (__builtin_amdgcn_classf(acc[u][r], INF_NAN) ||
+                                                           (__builtin_amdgcn_classf(acc[u][r], PLUS_ZERO) && last != 0)));
                         }
                     }
-                    if (__any(bad)) {
-                        acc[u] = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
-#pragma unroll 1
-                        for (int i0 = 0; i0 < nt; i0 += ATT_VC) {
-                            v4f wt[ATT_VC], vt[ATT_VC];
+                    again[u] = __any(bad);
+                    any = any || again[u];
+                }
+                if (any) {
 #pragma unroll
-                            for (int k = 0; k < ATT_VC; ++k) {
-                                wt[k] = s_load(min(i0 + k, nt - 1), u, lx);
+                    for (int u = 0; u < NP; ++u)
+                        if (again[u]) acc[u] = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll 1
+                    for (int i0 = 0; i0 < nt; i0 += ATT_VC) {
+                        v4f wt[NP][ATT_VC], vt[ATT_VC];
+#pragma unroll
+                        for (int k = 0; k < ATT_VC; ++k) {
+#pragma unroll
+                            for (int u = 0; u < NP; ++u) wt[u][k] = s_load(min(i0 + k, nt - 1), u, lx);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                vt[k][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                    vr, (int) ((uint32_t) (ATT_TILE * (i0 + k) + 4 * r + g4) * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0));
+                        }
+                        keep_order();
+#pragma unroll
+                        for (int k = 0; k < ATT_VC; ++k) {
+                            const int i = i0 + k;
+                            if (i >= nt) break;
+#pragma unroll
+                            for (int u = 0; u < NP; ++u) wt[u][k] = wt[u][k] * inv[u];
+                            if (i >= c0 && i < c1) {       // every pair attends to every key
 #pragma unroll
                                 for (int r = 0; r < 4; ++r)
-                                    vt[k][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                                        vr, (int) ((uint32_t) (ATT_TILE * (i0 + k) + 4 * r + g4) * 256u + (uint32_t) (16 * w + pi) * 4u), 0, 0));
+#pragma unroll
+                                    for (int u = 0; u < NP; ++u)
+                                        if (again[u]) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[u][k][r], vt[k][r], acc[u], 0, 0, 0);
+                                continue;
                             }
-                            keep_order();
 #pragma unroll
-                            for (int k = 0; k < ATT_VC; ++k) {
-                                const int i = i0 + k;
-                                if (i >= nt) break;
-                                wt[k] = wt[k] * inv[u];
-                                if (i >= c0 && i < c1) {   // every pair attends to every key
-#pragma unroll
-                                    for (int r = 0; r < 4; ++r)
-                                        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[k][r], vt[k][r], acc[u], 0, 0, 0);
-                                    continue;
-                                }
+                            for (int u = 0; u < NP; ++u) {
+                                if (!again[u]) continue;
 #pragma unroll 1
                                 for (int j = 0; j < ATT_TILE; ++j) {
                                     const int r = j >> 2, key = kl + ATT_TILE * i + j;
                                     const bool mine = (j & 3) == g4;
-                                    const float wj = r < 2 ? (r == 0 ? wt[k].x : wt[k].y) : (r == 2 ? wt[k].z : wt[k].w);
-                                    const float vj = r < 2 ? (r == 0 ? vt[k].x : vt[k].y) : (r == 2 ? vt[k].z : vt[k].w);
+                                    const v4f x = wt[u][k], y = vt[k];
+                                    const float wj = r < 2 ? (r == 0 ? x.x : x.y) : (r == 2 ? x.z : x.w);
+                                    const float vj = r < 2 ? (r == 0 ? y.x : y.y) : (r == 2 ? y.z : y.w);
                                     const v4f one = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? wj : 0.0f, mine ? vj : -0.0f, acc[u], 0, 0, 0);
                                     const uint64_t in = __ballot(act[u] && key >= lo[u] && key < hi[u]);
 #pragma unroll
@@ -1619,13 +1635,15 @@ __global__ __launch_bounds__(256, WS ? 2 : 4) void attention_mfma_kernel(attn_pa
                             }
                         }
                     }
+                }
+#pragma unroll
+                for (int u = 0; u < NP; ++u)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int pr = ATT_P * u + 4 * g4 + r;
-                        if (is_act(r))
+                        if (is_act(u, r))
                             p.out[(size_t) (t0 + (pr >> lg_rep)) * p.H * 64 + (size_t) ((g << lg_rep) + (pr & (rep - 1))) * 64 + 16 * w + pi] = acc[u][r];
                     }
-                }
             }
 #pragma unroll
             for (int u = 0; u < NP; ++u) todo[u] = todo[u] && !act[u];
